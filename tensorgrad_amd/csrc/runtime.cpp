@@ -195,6 +195,7 @@ struct Node {
   std::string shape;
   std::string detail;  // fused groups: member op kinds in program order
   bool ws = false;     // bind() reads cur_ws_ / cur_counters_ (rebound for the scratch-only step)
+  bool partials = false;   // reads column partials another launch of the step writes (in no tensor of `reads`)
   std::function<void(hipStream_t)> launch;   // bound after allocation
   std::function<std::function<void(hipStream_t)>()> bind;
 };
@@ -2714,7 +2715,8 @@ void Runtime::emit_colsums(const std::vector<int>& batch, bool with_scatter, boo
     const auto pt = colsum_part_.find(sop);
     const bool from_part = pt != colsum_part_.end();   // a GEMM epilogue's f64 partials
     const int64_t R = from_part ? pt->second.rows : c.R;
-    if (!from_part) n.reads.push_back(root(c.a));
+    if (from_part) n.partials = true;
+    else n.reads.push_back(root(c.a));
     if (c.b >= 0) n.reads.push_back(root(c.b));
     const int out = O(sop).at("out").i32();
     n.writes.push_back(root(out));
@@ -4312,7 +4314,8 @@ void Runtime::split_init_nodes() {
   for (auto& w : copy_writebacks_) pinned.insert(root(w.first));
   std::vector<Node> step;
   for (auto& n : nodes_) {
-    bool inv = n.kind != "adam_multi" && n.kind != "sgd_multi" && n.kind != "grad_norm" && !n.writes.empty();
+    bool inv = n.kind != "adam_multi" && n.kind != "sgd_multi" && n.kind != "grad_norm" && !n.partials &&
+               !n.writes.empty();
     for (int r : n.reads) if (!init_roots_.count(r)) inv = false;
     for (int w : n.writes) if (pinned.count(w)) inv = false;
     if (inv) {

@@ -309,6 +309,17 @@ def test_bias_sums_come_from_gemm_epilogues(monkeypatch):
     assert not [n for n in plain if 'colsum' in (n.get('ops') or '') or 'partials' in (n.get('ops') or '')]
 
 
+def test_bias_sums_from_partials_alone_run_every_step():
+    """At [16384, 129] every bias gradient of the small MLP comes from a GEMM epilogue's
+    column partials, so the launch that adds them reads no tensor: it is still a launch of
+    the step, not one of the constants computed once."""
+    ir = build_training_ir(configs.SinMLP(129), configs.sin_mlp_loss, {'x': [16384, 1], 'y': [16384, 1]},
+                           {'kind': 'adam', 'lr': 1e-3})
+    nodes = backend.plan(ir.wire_json())['nodes']
+    sums = [n for n in nodes if n['kind'] == 'reduce' and n['shape'] == '3 column sums']
+    assert len(sums) == 1 and sums[0]['ops'] == 'sum_partials,sum_partials,sum_partials'
+
+
 @pytest.mark.parametrize('n', [1, 3, 10])
 def test_forward_of_one_row_lowers_with_epilogues(n):
     """C1's forward at batch n (compileForward's shapes): every product is tiny and takes
