@@ -43,7 +43,7 @@ struct GemmArgs {
   int tiles_n, tiles_m;   // tile grid (per batch and split)
   float* out;             // split-K workspace (splits > 1)
   int64_t sOs, sOz;       // workspace strides (split, batch)
-  // Sum of products (SEG kernels): C = sum_s A_s B_s with K = nseg * seg_stages * BK, every
+  // Sum of products (SEG kernels): C = sum_s A_s B_s with K = nseg * seg_stages * (k of a stage), every
   // segment with its own operand bases and the strides of d (one batch, one split).
   int nseg = 1;
   int seg_stages = 0;
@@ -185,6 +185,111 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+template <int V>
+struct IntTag { static constexpr int value = V; };
+
+// The end of a tile: its accumulators (register r of lane l holds row (r / 4) * 8 + 4 (l / 32) + r % 4, column l % 32
+// of a 32 x 32 tile; the wavefront's tiles start at row mw, column nw) to the split-K workspace, or through the
+// epilogue. The block computed rows m0 .. m0 + BM and owns those from mlo <= .. on (below M; likewise columns): a tile
+// that lies whole inside the product takes the loops without a bound per element.
+template <int TM, int TN, int WGM, class Epi>
+__device__ __forceinline__ void tile_finish(const GemmArgs& g, const Epi& epi, f32x16 (&acc)[TM][TN], int64_t z0,
+                                            int64_t z1, int64_t zz, int split, uint32_t tm, int wrow, int lane,
+                                            int64_t mw, int64_t nw, int64_t mlo, int64_t nlo, int bm, int bn) {
+  const GemmDesc& d = g.d;
+  const int lrow = lane % 32, h = lane / 32;
+  auto finish = [&](auto edge_tag) {
+    constexpr bool EDGE = decltype(edge_tag)::value != 0;
+    auto row = [&](int i, int r) { return mw + i * 32 + (r / 4) * 8 + h * 4 + (r % 4); };
+    auto row_ok = [&](int64_t gm) { return !EDGE || (gm >= mlo && gm < d.M); };
+    auto col_ok = [&](int64_t gn) { return !EDGE || (gn >= nlo && gn < d.N); };
+    if (g.splits > 1) {   // split-K partial tile into the workspace
+      float* O = g.out + split * g.sOs + zz * g.sOz;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t gn = nw + j * 32 + lrow;
+          if (!col_ok(gn)) continue;
+          float* P = O + row(i, 0) * d.N + gn;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (row_ok(row(i, r))) P[((r / 4) * 8 + r % 4) * d.N] = acc[i][j][r];
+        }
+      return;
+    }
+    if constexpr (Epi::kPrefetch) {
+      // An epilogue that reads other tensors: every one of its loads for the wave's
+      // accumulator values is issued first (clamped to an element in range), then the values
+      // are computed and stored. Interleaved, each load would wait for the stores before it
+      // (the outputs may alias the inputs as far as the compiler knows): one memory latency
+      // per value.
+      typename Epi::Pre pre[TM][TN][16];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t gn = EDGE ? min((int64_t)(nw + j * 32 + lrow), d.N - 1) : nw + j * 32 + lrow;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) pre[i][j][r] = epi.load(d, EDGE ? min(row(i, r), d.M - 1) : row(i, r), gn);
+        }
+      if constexpr (Epi::kColSum) {
+        // The epilogue also returns the value of an output whose column sums are wanted: each
+        // lane totals its column over the wave's rows it holds (f64, in (i, r) order), the two
+        // lane halves (h = 0, 1: the other rows of the same column) are added, and lanes of
+        // h = 0 store the wave's partial row (one batch: z = 0).
+        double cs[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) cs[j] = 0.0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const int64_t gn = nw + j * 32 + lrow;
+            if (!col_ok(gn)) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              if (row_ok(row(i, r))) cs[j] += (double)epi(d, z0, z1, row(i, r), gn, acc[i][j][r], pre[i][j][r]);
+          }
+        const int64_t prow = (int64_t)tm * WGM + wrow;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const double t = cs[j] + __shfl_xor(cs[j], 32);
+          const int64_t gn = nw + j * 32 + lrow;
+          if (h == 0 && col_ok(gn)) g.colsum[prow * d.N + gn] = t;
+        }
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t gn = nw + j * 32 + lrow;
+          if (!col_ok(gn)) continue;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (row_ok(row(i, r))) epi(d, z0, z1, row(i, r), gn, acc[i][j][r], pre[i][j][r]);
+        }
+    } else {
+      float* C = d.C + z0 * d.sCz0 + z1 * d.sCz1;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t gn = nw + j * 32 + lrow;
+          if (!col_ok(gn)) continue;
+          float* P = C + row(i, 0) * d.sCm + gn * d.sCn;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (row_ok(row(i, r))) P[((r / 4) * 8 + r % 4) * d.sCm] = acc[i][j][r];
+        }
+    }
+  };
+  const int64_t r0 = (int64_t)tm * bm;   // the block's own first row; mlo is it, or where a shifted tile's part begins
+  if (mlo == r0 && r0 + bm <= d.M && nlo % bn == 0 && nlo + bn <= d.N) finish(IntTag<0>{});
+  else finish(IntTag<1>{});
 }
 
 // KG = 2 splits the k stages of a tile between two groups of four wavefronts by parity
@@ -418,107 +523,358 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint32_t b, const E
         for (int r = 0; r < 16; ++r) acc[i][j][r] += X[(((wave * TM + i) * TN + j) * 16 + r) * 64 + lane];
   }
 
-  if (g.splits > 1) {   // split-K partial tile into the workspace
-    float* O = g.out + split * g.sOs + zz * g.sOz;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t gn = n0 + wn0 + j * 32 + lrow;
-        if (gn >= d.N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t gm = m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-          if (gm < d.M) O[gm * d.N + gn] = acc[i][j][r];
-        }
-      }
-    return;
-  }
-  if constexpr (Epi::kPrefetch) {
-    // An epilogue that reads other tensors: every one of its loads for the wave's
-    // accumulator values is issued first (clamped to an element in range), then the values
-    // are computed and stored. Interleaved, each load would wait for the stores before it
-    // (the outputs may alias the inputs as far as the compiler knows): one memory latency
-    // per value.
-    typename Epi::Pre pre[TM][TN][16];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t gn = min((int64_t)(n0 + wn0 + j * 32 + lrow), d.N - 1);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t gm = min((int64_t)(m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4)), d.M - 1);
-          pre[i][j][r] = epi.load(d, gm, gn);
-        }
-      }
-    if constexpr (Epi::kColSum) {
-      // The epilogue also returns the value of an output whose column sums are wanted: each
-      // lane totals its column over the wave's rows it holds (f64, in (i, r) order), the two
-      // lane halves (h = 0, 1: the other rows of the same column) are added, and lanes of
-      // h = 0 store the wave's partial row (one batch: z = 0).
-      double cs[TN];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) cs[j] = 0.0;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t gn = n0 + wn0 + j * 32 + lrow;
-          if (gn >= d.N) continue;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int64_t gm = m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-            if (gm < d.M) cs[j] += (double)epi(d, z0, z1, gm, gn, acc[i][j][r], pre[i][j][r]);
-          }
-        }
-      const int64_t prow = (int64_t)tm * WGM + wave / WGN;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const double t = cs[j] + __shfl_xor(cs[j], 32);
-        const int64_t gn = n0 + wn0 + j * 32 + lrow;
-        if (h == 0 && gn < d.N) g.colsum[prow * d.N + gn] = t;
-      }
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t gn = n0 + wn0 + j * 32 + lrow;
-        if (gn >= d.N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t gm = m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-          if (gm < d.M) epi(d, z0, z1, gm, gn, acc[i][j][r], pre[i][j][r]);
-        }
-      }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t gn = n0 + wn0 + j * 32 + lrow;
-        if (gn >= d.N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t gm = m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
-          if (gm < d.M) epi(d, z0, z1, gm, gn, acc[i][j][r]);
-        }
-      }
-  }
+  tile_finish<TM, TN, WGM>(g, epi, acc, z0, z1, zz, split, tm, wave / WGN, lane, m0 + wm0, n0 + wn0, m0, n0, BM, BN);
 }
 
 // The plain epilogue: element (z, gm, gn) of the product to C.
-struct StoreC {
+struct StoreC {   // (tile_finish stores it)
   static constexpr bool kPrefetch = false;
   static constexpr bool kColSum = false;
-  __device__ __forceinline__ void operator()(const GemmDesc& d, int64_t z0, int64_t z1, int64_t gm, int64_t gn,
-                                             float v) const {
-    d.C[z0 * d.sCz0 + z1 * d.sCz1 + gm * d.sCm + gn * d.sCn] = v;
+};
+
+
+// ---- f32 products on the bf16 matrix cores ---------------------------------------------
+// The bf16 MFMAs run at 16 times the f32 rate. An f32 value is exactly the sum of three bf16 values (round to nearest,
+// then the same of what is left, twice: 8 + 8 + 8 bits), so a product is nine bf16 products, of which the three below
+// 2^-25 of the largest (mid * low, low * mid, low * low) are left out: six MFMAs in place of sixteen's worth of time.
+// Accuracy against 64 bits is no worse than the f32 tile's (norm-wise, K = 256 .. 4096: 0.9e-7 .. 2.3e-7 against
+// 1.2e-7 .. 2.3e-7): the products are exact, an MFMA adds 16 of them with one rounding where the f32 one adds two, and
+// every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum.
+// Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
+// are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile.
+//
+// What bounds it: per 16 k a wavefront with a 64 x 64 tile issues 24 MFMAs (32 cycles each) and about 130 vector
+// instructions (5.5 per element split, 2 per accumulator), and an MFMA keeps the vector port for half its time, so the
+// two together need about 1.4 of the MFMAs' own time; two blocks a CU hide each other's barriers and latencies. At
+// 4096^3 the matrix cores are 59 % busy at the 1.8 GHz the card then holds (187 TFLOP/s as f32 work, against 130 for
+// the f32 tile); [65536, 256] x [256, 256] 92 -> 58 us, [4000, 512] x [512, 2048] 88 -> 55 us.
+//
+// Tile: operands go through registers (loads three stages ahead of their use, split, then stored as three bf16 planes
+// into the other half of a double LDS buffer while this half is multiplied), so they need no alignment: a load is
+// 16 bytes along k (k-contiguous operand) or 8 bytes along the rows (row-contiguous), from any 4-byte boundary.
+// Nothing is read out of range and nothing is clamped: a tile that would pass the last row starts BM rows before it
+// instead (and stores only its own rows), and a K that is no multiple of 16 starts with a stage that overlaps the next
+// one, the overlap zeroed. So it needs M >= BM, N >= BN and 16 or more k per split.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+
+// Two values as pairs of their three bf16 terms.
+__device__ __forceinline__ void split3(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = bf16_pair(x0, x1);
+  const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+  m = bf16_pair(r0, r1);
+  const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
+  l = bf16_pair(s0, s1);
+}
+
+constexpr int kXK = 16;   // k of a stage: one MFMA's
+
+// One operand's ROWS x 16 stage for 256 threads. In LDS a plane is rows of 32 bytes whose two 16-byte chunks (8 k each)
+// are swapped by a function of the row, so the fragment reads (a lane's 8 k of its row) meet no bank twice; rows of a
+// row-contiguous operand are stored evens first, which spreads the stores of its threads (two neighbouring rows each).
+template <int ROWS, bool KFAST>
+struct XTile {
+  static constexpr int NT = 256;
+  static constexpr int PLANE = ROWS * 32;          // bytes
+  static constexpr int SIZE = 3 * PLANE;
+  static constexpr int PER = ROWS * kXK / NT;      // floats per thread
+  static constexpr int PK = PER / 2;               // row-contiguous: a thread's patch is 2 rows x PK k
+  static_assert(PER == 4 || PER == 8, "64 or 128 rows");
+
+  __device__ __forceinline__ static int at(int row, int c) {   // byte offset of chunk c of a row
+    if (KFAST) return row * 32 + ((c ^ (row >> 2) ^ (row >> 3)) & 1) * 16;
+    const int p = (row >> 1) + (row & 1) * (ROWS / 2);
+    return p * 32 + ((c ^ row ^ (p >> 2)) & 1) * 16;
+  }
+  // Byte offset of a thread's first load from the stage's origin, and the (uniform) distance to its next.
+  __device__ __forceinline__ static uint32_t first(int64_t sr, int64_t sk, int tid) {
+    if (KFAST) return (uint32_t)((tid >> 2) * (int)sr + (tid & 3) * 4) * 4u;
+    return (uint32_t)((tid % (ROWS / 2)) * 2 + (tid / (ROWS / 2)) * PK * (int)sk) * 4u;
+  }
+  __device__ __forceinline__ static uint32_t step(int64_t sr, int64_t sk) {
+    return KFAST ? (uint32_t)(NT / 4 * (int)sr) * 4u : (uint32_t)sk * 4u;
+  }
+  __device__ __forceinline__ static void load(float* q, const float* X, uint32_t off, uint32_t stp) {
+    const char* x = reinterpret_cast<const char*>(X);
+    if (KFAST) {
+#pragma unroll
+      for (int e = 0; e < PER / 4; ++e) {
+        const f32x4u v = *reinterpret_cast<const f32x4u*>(x + (uint64_t)(e * stp) + off);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[e * 4 + u] = v[u];
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < PK; ++u) {
+        const f32x2u v = *reinterpret_cast<const f32x2u*>(x + (uint64_t)(u * stp) + off);
+        q[u] = v[0];
+        q[PK + u] = v[1];
+      }
+    }
+  }
+  // Zero the k of a stage at and past `keep`.
+  __device__ __forceinline__ static void mask(float* q, int keep, int tid) {
+    const int k0 = KFAST ? (tid & 3) * 4 : (tid / (ROWS / 2)) * PK;
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (k0 + (KFAST ? e % 4 : e % PK) >= keep) q[e] = 0.0f;
+  }
+  __device__ __forceinline__ static void put(char* p, const uint32_t* v, int n) {
+    if (n == 2) *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
+    else *reinterpret_cast<uint32_t*>(p) = v[0];
+  }
+  __device__ __forceinline__ static void store(const float* q, char* L, int tid) {
+    constexpr int W = KFAST ? 2 : PK / 2;          // pairs of k in a unit
+    constexpr int UNITS = KFAST ? PER / 4 : 2;
+#pragma unroll
+    for (int e = 0; e < UNITS; ++e) {
+      const int row = KFAST ? (tid >> 2) + e * (NT / 4) : (tid % (ROWS / 2)) * 2 + e;
+      const int k = KFAST ? (tid & 3) * 4 : (tid / (ROWS / 2)) * PK;
+      uint32_t h[W], m[W], l[W];
+#pragma unroll
+      for (int u = 0; u < W; ++u) split3(q[(e * W + u) * 2], q[(e * W + u) * 2 + 1], h[u], m[u], l[u]);
+      char* p = L + at(row, k >> 3) + (k & 7) * 2;
+      put(p, h, W);
+      put(p + PLANE, m, W);
+      put(p + 2 * PLANE, l, W);
+    }
+  }
+  __device__ __forceinline__ static bf16x8 frag(const char* L, int plane, int row, int h) {
+    return *reinterpret_cast<const bf16x8*>(L + plane * PLANE + at(row, h));
   }
 };
 
+// One output tile (tile number b of the problem g) by KG groups of four wavefronts, each over its own share of the k
+// stages (a small grid then still puts several wavefronts on a SIMD); the groups' sums are added in order.
+// SEG: a sum of products, k segment after k segment, each of whole stages (GemmArgs::seg_stages, in 16 k).
+// CAT: A is a concatenation along k of d.A (whole stages) and g.catA (cat_k1 >= 16 of any number), catA's part first.
+template <int BM, int BN, bool AK, bool BKF, int KG, class Epi, bool SEG = false, bool CAT = false>
+__device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi& epi) {
+  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;   // wavefronts 2 x 2
+  using TA = XTile<BM, AK>;
+  using TB = XTile<BN, BKF>;
+  constexpr int BUF = TA::SIZE + TB::SIZE;
+  static_assert(!(SEG && CAT) && (!CAT || AK), "CAT: a k-contiguous A");
+  static_assert((KG - 1) * TM * TN * 16 * 256 * 4 <= KG * 2 * BUF, "the groups' exchange fits the buffers");
+  __shared__ __attribute__((aligned(16))) char lds[KG * 2 * BUF];
+  const GemmDesc& d = g.d;
+  const int tid = threadIdx.x % 256, lane = tid & 63;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave / 2) * WM, wn0 = (wave % 2) * WN;
+  const uint32_t tn = b % g.tiles_n, rest = b / g.tiles_n, tm = rest % g.tiles_m, zs = rest / g.tiles_m;
+  const int64_t mlo = (int64_t)tm * BM, nlo = (int64_t)tn * BN;        // the tile's own first row and column
+  const int64_t m0 = min(mlo, d.M - BM), n0 = min(nlo, d.N - BN);      // the first ones it computes
+  const int64_t zz = zs / g.splits;
+  const int split = zs % g.splits;
+  const int64_t z0 = zz / d.bdiv, z1 = zz % d.bdiv;
+  const float* A = d.A + z0 * d.sAz0 + z1 * d.sAz1 + m0 * d.sAm;
+  const float* B = d.B + z0 * d.sBz0 + z1 * d.sBz1 + n0 * d.sBn;
+  const int64_t kbeg = split * g.k_per_split, kend = min(d.K, kbeg + g.k_per_split);
+  // CAT (one split): the second source's cat_k1 first, in n1 stages
+  const int k1 = CAT ? (int)(d.K - (int64_t)g.cat_stages * kXK) : 0;
+  const int n1 = CAT ? (k1 + kXK - 1) / kXK : 0;
+  const int nst = CAT ? n1 + g.cat_stages : (int)((kend - kbeg + kXK - 1) / kXK);
+  // the first stage's k that the second does not cover
+  const int keep = CAT ? k1 - (n1 - 1) * kXK : (int)(kend - kbeg) - (nst - 1) * kXK;
+  const int s0 = (int)((int64_t)kg * nst / KG), cnt = (int)((int64_t)(kg + 1) * nst / KG) - s0;   // the group's stages
+  const int most = (nst + KG - 1) / KG;
+  const uint32_t offa = TA::first(d.sAm, d.sAk, tid), offb = TB::first(d.sBn, d.sBk, tid);
+  const uint32_t stpa = TA::step(d.sAm, d.sAk), stpb = TB::step(d.sBn, d.sBk);
+  const uint32_t offc = CAT ? TA::first(g.catAm, 1, tid) : 0, stpc = CAT ? TA::step(g.catAm, 1) : 0;
+  float qa[2][TA::PER], qb[2][TB::PER];
+  // stage st (of all) into register set `set`; stage 0 starts at the range's begin, the others end at its end
+  auto load = [&](int st, int set) {
+    if (SEG) {
+      const int ss = g.seg_stages;
+      const int sg = (st >= ss) + (st >= 2 * ss) + (st >= 3 * ss);   // (at most kMaxSeg = 4; no division per stage)
+      const int64_t k = (int64_t)(st - sg * ss) * kXK;
+      const float* sa = sg == 0 ? g.segA[0] : sg == 1 ? g.segA[1] : sg == 2 ? g.segA[2] : g.segA[3];
+      const float* sb = sg == 0 ? g.segB[0] : sg == 1 ? g.segB[1] : sg == 2 ? g.segB[2] : g.segB[3];
+      TA::load(qa[set], sa + m0 * d.sAm + k * d.sAk, offa, stpa);
+      TB::load(qb[set], sb + n0 * d.sBn + k * d.sBk, offb, stpb);
+    } else if (CAT) {
+      const bool second = st < n1;
+      const int64_t k = second ? (st == 0 ? 0 : k1 - (int64_t)(n1 - st) * kXK) : (int64_t)(st - n1) * kXK;
+      const float* a = second ? g.catA + m0 * g.catAm + k : A + k;
+      TA::load(qa[set], a, second ? offc : offa, second ? stpc : stpa);
+      TB::load(qb[set], B + ((second ? (int64_t)g.cat_stages * kXK : 0) + k) * d.sBk, offb, stpb);
+    } else {
+      const int64_t k = st == 0 ? kbeg : kend - (int64_t)(nst - st) * kXK;
+      TA::load(qa[set], A + k * d.sAk, offa, stpa);
+      TB::load(qb[set], B + k * d.sBk, offb, stpb);
+    }
+  };
+  auto ahead = [&](int st, int set) { load(s0 + min(st, cnt - 1), set); };   // past the last stage: the last again
+  auto meet = [&]() {   // LDS traffic only: the loads of later stages stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  char* mine = lds + kg * 2 * BUF;
+  f32x16 acc[TM][TN], part[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = part[i][j][r] = 0.0f;
+  const int lrow = lane % 32, h = lane / 32;
+  // The stage in buffer P is multiplied while the next is split into the other buffer and the third from here loaded.
+  // FRESH: the running sums take the last stages' part and a new one begins.
+  auto body = [&](int st, auto ptag, auto ftag) {
+    constexpr int P = decltype(ptag)::value;
+    constexpr bool FRESH = decltype(ftag)::value != 0;
+    const char *La = mine + P * BUF, *Lb = La + TA::SIZE;
+    // terms, small ones first: (hi, low) (low, hi) (mid, mid) (hi, mid) (mid, hi) (hi, hi)
+    constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};
+    constexpr int OA[3] = {0, 2, 1}, OB[3] = {2, 0, 1};   // planes in the order of their first use
+    bf16x8 a[3][TM], bb[3][TN];
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[OA[o]][i] = TA::frag(La, OA[o], wm0 + i * 32 + lrow, h);
+      bb[OB[o]][0] = TB::frag(Lb, OB[o], wn0 + lrow, h);
+    }
+#pragma unroll
+    for (int j = 1; j < TN; ++j)
+#pragma unroll
+      for (int o = 0; o < 3; ++o) bb[OB[o]][j] = TB::frag(Lb, OB[o], wn0 + j * 32 + lrow, h);
+    TA::store(qa[P ^ 1], mine + (P ^ 1) * BUF, tid);
+    TB::store(qb[P ^ 1], mine + (P ^ 1) * BUF + TA::SIZE, tid);
+    ahead(st + 3, P ^ 1);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if (FRESH) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] += part[i][j];
+      }
+#pragma unroll
+      for (int t = 0; t < 6; ++t)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const f32x16 c = FRESH && t == 0 ? (f32x16)(0.0f) : part[i][j];
+          part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t]][i], bb[PB[t]][j], c, 0, 0, 0);
+        }
+    }
+    meet();
+  };
+  if (cnt > 0) {
+    load(s0, 0);
+    if (s0 == 0 && keep < kXK) {
+      TA::mask(qa[0], keep, tid);
+      TB::mask(qb[0], keep, tid);
+    }
+    ahead(1, 1);
+    TA::store(qa[0], mine, tid);
+    TB::store(qb[0], mine + TA::SIZE, tid);
+    ahead(2, 0);
+  }
+  meet();
+  for (int st = 0; st < most; st += 2) {   // the barriers are the whole block's: every group passes `most`
+    if (st < cnt) body(st, IntTag<0>{}, IntTag<1>{});
+    else meet();
+    if (st + 1 >= most) break;
+    if (st + 1 < cnt) body(st + 1, IntTag<1>{}, IntTag<0>{});
+    else meet();
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] += part[i][j];
+  if (KG > 1) {
+    float* X = reinterpret_cast<float*>(lds);   // every group has passed its last read of the buffers
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            X[((((kg - 1) * 4 + wave) * TM * TN + i * TN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] += X[(((q * 4 + wave) * TM * TN + i * TN + j) * 16 + r) * 64 + lane];
+  }
+  // 0 * v is 0 for a finite v and NaN otherwise
+  float bad = 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad = fmaf(acc[i][j][r], 0.0f, bad);
+  if (__builtin_amdgcn_ballot_w64(bad != 0.0f) != 0) {
+    // x3_redo: the wavefront's tiles again on f32 MFMAs (the sums of k = 0, 1, 0, 1 .. lane halves, a fresh accumulator
+    // per 32 k), straight from global memory. Rare, so plain.
+    const int len = (int)(kend - kbeg);
+    const int segk = SEG ? g.seg_stages * kXK : 0, k0cat = CAT ? g.cat_stages * kXK : 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int kb = 0; kb < len; kb += 32) {
+      f32x16 sum[TM][TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sum[i][j][r] = 0.0f;
+#pragma unroll 1
+      for (int u = 0; u < 32; u += 2) {
+        const int k = kb + u + h, kc = min(k, len - 1);
+        const float *pa = A + (kbeg + kc) * d.sAk, *pb = B + (kbeg + kc) * d.sBk;
+        int64_t sam = d.sAm;
+        if (SEG) {
+          const int sg = min(kb + u, len - 1) / segk;   // whole segments of 16 k: the same for both lane halves
+          const int64_t ks = kc - sg * segk;
+          const float* sa = sg == 0 ? g.segA[0] : sg == 1 ? g.segA[1] : sg == 2 ? g.segA[2] : g.segA[3];
+          const float* sb = sg == 0 ? g.segB[0] : sg == 1 ? g.segB[1] : sg == 2 ? g.segB[2] : g.segB[3];
+          pa = sa + m0 * d.sAm + ks * d.sAk;
+          pb = sb + n0 * d.sBn + ks * d.sBk;
+        }
+        if (CAT && kc >= k0cat) {
+          pa = g.catA + m0 * g.catAm + (kc - k0cat);
+          sam = g.catAm;
+        }
+        float av[TM], bv[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) av[i] = k < len ? pa[(wm0 + i * 32 + lrow) * sam] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bv[j] = k < len ? pb[(wn0 + j * 32 + lrow) * d.sBn] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], sum[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += sum[i][j];
+    }
+  }
+  tile_finish<TM, TN, 2>(g, epi, acc, z0, z1, zz, split, tm, wave / 2, lane, m0 + wm0, n0 + wn0, mlo, nlo, BM, BN);
+}
 
 // ---- skinny products (the layout and the choice are described in k_gemm.hip) ----------
 // GemmArgs as: tiles_m = row blocks of 16, tiles_n = column blocks of NT x 16, splits and

@@ -357,7 +357,8 @@ JitKernel gemm_epi_kernel(const FusedProgram& p, const FusedInstr* code, const G
   if (c.colsum_out >= 0) o << I << "return tgk::bitsf(" << R(p.out_reg[c.colsum_out]) << ");\n";
   else o << I << "return 0.0f;\n";
   o << "  }\n};\n}  // namespace\n";
-  o << "extern \"C\" __global__ void __launch_bounds__(" << c.nt
+  // (the split-bf16 tile: 256 registers, two blocks of a 128 x 128 tile a CU)
+  o << "extern \"C\" __global__ void __launch_bounds__(" << c.nt << (c.x3 ? ", 2" : "")
     << ") @NAME@(const tgk::gd::GemmArgs g, const tgk::JitArgs A) {\n";
   o << "  const @NAME@_epi e{A, " << (dropout ? "A.seed ? (unsigned)*A.seed : 0u" : "0u") << "};\n";
   if (c.skinny) {
@@ -368,6 +369,10 @@ JitKernel gemm_epi_kernel(const FusedProgram& p, const FusedInstr* code, const G
     o << "  tgk::gd::tiny_tile<" << c.bm << ">(g, e);\n}\n";
   } else if (c.smallk) {
     o << "  tgk::gd::smallk_tile<" << c.bm << ", " << c.bk << ">(g, e);\n}\n";
+  } else if (c.x3) {
+    o << "  tgk::gd::x3_tile<" << c.bm << ", " << c.bn << ", " << (c.ak ? "true" : "false") << ", "
+      << (c.bkf ? "true" : "false") << ", " << c.kg << ", @NAME@_epi, false, " << (c.cat ? "true" : "false")
+      << ">(g, tgk::gd::xcd_order(blockIdx.x, gridDim.x), e);\n}\n";
   } else {
     o << "  tgk::gd::gemm_tile<" << c.bm << ", " << c.bn << ", " << c.bk << ", " << c.ns << ", "
       << (c.ak ? "true" : "false") << ", " << (c.bkf ? "true" : "false") << ", " << c.nt << ", " << c.kg;

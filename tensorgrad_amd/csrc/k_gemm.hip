@@ -1,4 +1,5 @@
-// f32 GEMM on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
+// f32 GEMM on the gfx950 matrix cores: products of 64 or more rows and columns and 32 or more k as
+// split-bf16 MFMAs (x3_tile, gemm_dev.h), the rest on v_mfma_f32_32x32x2_f32, described here.
 //
 // C[z][m][n] = sum_k A[z][m][k] * B[z][k][n] with arbitrary element strides, so the IR's
 // transposes (swapAxes before matmul, splitHeads / mergeHeads permutes) are read in place
@@ -260,6 +261,27 @@ __global__ __launch_bounds__(NT) void k_gemm_dma_group(const GemmArgs* __restric
   gemm_tile<BM, BN, BK, NS, AK, BKF, NT, KG>(g, b - starts[p], StoreC{});
 }
 
+// The split-bf16 tile (x3_tile). Registers: two blocks a CU of the 128 x 128 tile, three of the 128 x 64 ones, four of
+// four wavefronts of the 64 x 64 tile.
+constexpr int x3_waves(int BM, int BN) { return BM * BN == 128 * 128 ? 2 : BM * BN == 128 * 64 ? 3 : 4; }
+
+template <int BM, int BN, bool AK, bool BKF, int KG, bool SEG = false, bool CAT = false>
+__global__ __launch_bounds__(256 * KG, x3_waves(BM, BN)) void k_gemm_x3(GemmArgs g) {
+  x3_tile<BM, BN, AK, BKF, KG, StoreC, SEG, CAT>(g, xcd_order(blockIdx.x, gridDim.x), StoreC{});
+}
+
+template <int BM, int BN, bool AK, bool BKF, int KG>
+__global__ __launch_bounds__(256 * KG, x3_waves(BM, BN)) void k_gemm_x3_group(const GemmArgs* __restrict__ table,
+                                                                                const uint32_t* __restrict__ starts,
+                                                                                int n) {
+  const uint32_t b = xcd_order(blockIdx.x, gridDim.x);
+  int p = 0;
+  for (int q = 1; q < n; ++q)
+    if (starts[q] <= b) p = q;
+  const GemmArgs g = table[p];
+  x3_tile<BM, BN, AK, BKF, KG, StoreC>(g, b - starts[p], StoreC{});
+}
+
 // Sum split-K partials in split order into C (eight partial loads in flight per thread).
 __global__ void k_splitk_reduce(const float* __restrict__ work, int splits, int64_t sOs, GemmDesc d) {
   const int64_t MN = d.M * d.N, total = MN * d.batch;
@@ -313,6 +335,105 @@ Plan plan_for(const GemmDesc& d) {
     }
   }
   return p;
+}
+
+// The split-bf16 tile takes every product of 64 or more rows and columns and 32 or more k whose operands have a unit
+// stride along k or along their rows (from any address); offsets within a tile stay below 2^31 bytes.
+bool x3_ok(const GemmDesc& d) {
+  if (d.M < 64 || d.N < 64 || d.K < 32 || d.batch <= 0) return false;
+  const bool ak = d.sAk == 1, bk = d.sBk == 1 && d.sBn != 1;
+  if ((!ak && d.sAm != 1) || (!bk && d.sBn != 1)) return false;
+  const int64_t sa = ak ? d.sAm : d.sAk, sb = bk ? d.sBn : d.sBk, lim = (int64_t(1) << 31) / (128 * 4);
+  return sa >= 0 && sb >= 0 && sa < lim && sb < lim && d.K < (int64_t(1) << 31);
+}
+
+// Time of a 16-k stage in us of the `on_cu` groups of wavefronts that share a CU, each with a tile (or, kg of them, a
+// share of one's stages): `alone` for one, `more` for each other while they hide each other's latencies, `full` per
+// group at least (measured over 4096^3, [4096, 256] x [256, 1024], [512, 4000] x [4000, 2048], [1600, 1536] x
+// [1536, 512]). A small tile's stages take longer per output; a CU with one large tile waits for its barriers.
+struct XTiling { int bm, bn, kg; double alone, more, full; };
+constexpr XTiling kXTilings[] = {{128, 128, 1, 0.79, 0.63, 0.71}, {128, 128, 2, 0.79, 0.63, 0.71},
+                                 {128, 64, 1, 0.57, 0.30, 0.42},  {128, 64, 2, 0.57, 0.30, 0.42},
+                                 {64, 128, 1, 0.57, 0.30, 0.42},  {64, 128, 2, 0.57, 0.30, 0.42},
+                                 {64, 64, 1, 0.43, 0.19, 0.25},   {64, 64, 2, 0.43, 0.19, 0.25},
+                                 {64, 64, 4, 0.43, 0.19, 0.25}};
+constexpr int kXTilingCount = sizeof(kXTilings) / sizeof(kXTilings[0]);
+
+double x3_time(const XTiling& t, int64_t tiles, int64_t splits, int64_t k) {
+  const int64_t on_cu = (tiles * splits + 255) / 256 * t.kg;   // groups on the fullest CU
+  const int64_t stages = ((k + splits - 1) / splits + 16 * t.kg - 1) / (16 * t.kg);
+  // the groups' exchange and the larger block's launch: [1024, 64] x [64, 64] 4.7 us by one group, 6.9 by four
+  const double meet = t.kg == 4 ? 2.8 : t.kg == 2 ? 1.0 : 0.0;
+  return meet + stages * std::max(t.alone + (on_cu - 1) * t.more, on_cu * t.full);
+}
+
+int64_t x3_tiles(const XTiling& t, const GemmDesc& d) {
+  return (d.M + t.bm - 1) / t.bm * ((d.N + t.bn - 1) / t.bn) * d.batch;
+}
+
+// Longest k range that one group sums: the running sum of a range takes an addition per 32 k, the f32 tiles' (two
+// running sums over each split of plan_for) one per 64 or 128. Error variance against 64 bits, in units of 1e-14:
+// 0.5 + 1.2e-3 k here, 1.15 + 0.52e-3 k there; this keeps the first below the second.
+int64_t x3_range(const GemmDesc& d) { return 512 + (int64_t)(0.4 * (double)plan_for(d).kps); }
+
+struct XPlan { int tiling, splits; int64_t kps; double us; };
+
+// Split-K partials of a product stay under this, so that a step's scratch (with its launch counters) fits the
+// library's static array.
+constexpr int64_t kXSplitBytes = (16 << 20) - (512 << 10);
+
+// The tiling (and for K >= 1024 the split of K, partial products added by k_splitk_reduce) with the least time by the
+// figures above. A product with K under 1024 is never split, so its epilogue group can run in it.
+XPlan x3_plan(const GemmDesc& d) {
+  XPlan best{-1, 1, d.K, 0.0};
+  const int64_t range = x3_range(d);
+  for (int t = 0; t < kXTilingCount; ++t) {
+    const XTiling& x = kXTilings[t];
+    if (d.M < x.bm || d.N < x.bn) continue;
+    const int64_t tiles = x3_tiles(x, d);
+    for (int64_t s = 1; s <= 64; ++s) {
+      if (s > 1 && (d.K < 1024 || d.K / s < 256 || s * d.M * d.N * d.batch * 4 > kXSplitBytes)) break;
+      int64_t kps = (d.K + s - 1) / s;
+      if (s > 1) kps = (kps + kXK - 1) / kXK * kXK;
+      const int splits = (int)((d.K + kps - 1) / kps);
+      if (d.K - (splits - 1) * kps < kXK) continue;   // every split has a whole stage
+      const bool fits = kps <= range * x.kg;
+      double us = x3_time(x, tiles, splits, d.K);
+      if (splits > 1) us += 5.0 + (double)splits * d.M * d.N * d.batch * 8 / 4e6;   // the partials' way and their sum
+      if (best.tiling < 0 || (fits && us < best.us)) best = {t, splits, kps, fits ? us : 1e30};
+    }
+  }
+  return best;
+}
+
+// One tiling for several unsplit products in one launch; its time in us.
+int x3_group_tiling(const GemmDesc* ds, int n, double* us_out) {
+  int best = -1;
+  double best_us = 0.0;
+  // Together these fill the chip with 64 x 64 tiles of one running sum over all of K: the f32 tiles' error then has
+  // variance 1.1 + 0.97e-3 k (x3_range), which allows longer ranges.
+  int64_t t64 = 0;
+  for (int q = 0; q < n; ++q) t64 += (ds[q].M + 63) / 64 * ((ds[q].N + 63) / 64) * ds[q].batch;
+  auto range = [&](const GemmDesc& d) {
+    return t64 >= 512 && d.K > kShortK ? std::max(x3_range(d), 512 + (int64_t)(0.75 * (double)d.K)) : x3_range(d);
+  };
+  for (int t = 0; t < kXTilingCount; ++t) {
+    const XTiling& x = kXTilings[t];
+    int64_t tiles = 0, kmax = 0, work = 0;
+    bool fits = true;
+    for (int q = 0; q < n; ++q) {
+      fits = fits && ds[q].M >= x.bm && ds[q].N >= x.bn && ds[q].K <= range(ds[q]) * x.kg;
+      tiles += x3_tiles(x, ds[q]);
+      work += x3_tiles(x, ds[q]) * ds[q].K;
+      kmax = std::max(kmax, ds[q].K);
+    }
+    if (!fits && !(x.bm == 64 && x.bn == 64 && x.kg == 4)) continue;   // (the one that takes them all)
+    // the launch ends with its longest tile; short ones fill in beside it
+    const double us = std::max(x3_time(x, 1, 1, kmax), x3_time(x, tiles, 1, (work + tiles - 1) / tiles));
+    if (best < 0 || us < best_us) { best = t; best_us = us; }
+  }
+  if (us_out) *us_out = best_us;
+  return best;
 }
 
 // Conditions of the direct-to-LDS kernel: whole BK stages in every split, 16-byte aligned
@@ -456,8 +577,8 @@ int64_t gemm_workspace_floats(const GemmDesc& d) {
   if (!gemm_is_tiny(d) && gemm_is_smallk(d)) return 0;
   SkinnyPlan sk;
   if (!gemm_is_tiny(d) && skinny_plan(d, sk)) return sk.splits > 1 ? (int64_t)sk.splits * d.M * d.N : 0;
-  Plan p = plan_for(d);
-  return p.splits > 1 ? (int64_t)p.splits * d.batch * d.M * d.N : 0;
+  const int splits = x3_ok(d) ? x3_plan(d).splits : plan_for(d).splits;
+  return splits > 1 ? (int64_t)splits * d.batch * d.M * d.N : 0;
 }
 
 namespace {
@@ -508,6 +629,23 @@ static int64_t tiny_blocks(const GemmDesc& d, int L) {
 bool gemm_is_tiny(const GemmDesc& d) {
   return d.M > 0 && d.N > 0 && d.K > 0 && d.batch > 0 && (d.M == 1 || d.N == 1 || d.K == 1) &&
          d.M * d.N <= kTinyMacs && d.K <= kTinyMacs && d.M * d.N * d.K * d.batch <= kTinyMacs;
+}
+
+// The launch of d's plan on the split-bf16 tile (x3_ok).
+static GemmArgs x3_args(const GemmDesc& d, float* work, XPlan& xp, int64_t& blocks) {
+  xp = x3_plan(d);
+  const XTiling& t = kXTilings[xp.tiling];
+  GemmArgs g{d, xp.kps, xp.splits, 0, 0, nullptr, 0, 0};
+  if (xp.splits > 1) {
+    g.out = work;
+    g.sOz = d.M * d.N;
+    g.sOs = d.batch * d.M * d.N;
+  }
+  g.tiles_n = (int)((d.N + t.bn - 1) / t.bn);
+  g.tiles_m = (int)((d.M + t.bm - 1) / t.bm);
+  blocks = (int64_t)g.tiles_n * g.tiles_m * d.batch * xp.splits;
+  if (blocks >= (int64_t(1) << 31)) throw std::runtime_error("gemm: too many tiles");
+  return g;
 }
 
 void gemm(const GemmDesc& d, float* work, hipStream_t st) {
@@ -565,6 +703,38 @@ void gemm(const GemmDesc& d, float* work, hipStream_t st) {
     }
     return;
   }
+  auto add_splits = [&](int splits) {
+    const int64_t total = d.batch * d.M * d.N;
+    const int64_t nb = std::min<int64_t>((total + 255) / 256, 4096);
+    klaunch(k_splitk_reduce, (int)nb, 256, 0, st, work, splits, total, d);
+  };
+  if (x3_ok(d)) {
+    int64_t blocks = 0;
+    XPlan xp;
+    const GemmArgs g = x3_args(d, work, xp, blocks);
+    const bool ak = d.sAk == 1, bk = d.sBk == 1 && d.sBn != 1;
+#define TG_X3_LAUNCH(BM_, BN_, KG_)                                                                                   \
+  do {                                                                                                                \
+    if (ak && bk) klaunch(k_gemm_x3<BM_, BN_, true, true, KG_>, (unsigned)blocks, 256 * KG_, 0, st, g);               \
+    else if (ak) klaunch(k_gemm_x3<BM_, BN_, true, false, KG_>, (unsigned)blocks, 256 * KG_, 0, st, g);               \
+    else if (bk) klaunch(k_gemm_x3<BM_, BN_, false, true, KG_>, (unsigned)blocks, 256 * KG_, 0, st, g);               \
+    else klaunch(k_gemm_x3<BM_, BN_, false, false, KG_>, (unsigned)blocks, 256 * KG_, 0, st, g);                      \
+  } while (0)
+    switch (xp.tiling) {
+      case 0: TG_X3_LAUNCH(128, 128, 1); break;
+      case 1: TG_X3_LAUNCH(128, 128, 2); break;
+      case 2: TG_X3_LAUNCH(128, 64, 1); break;
+      case 3: TG_X3_LAUNCH(128, 64, 2); break;
+      case 4: TG_X3_LAUNCH(64, 128, 1); break;
+      case 5: TG_X3_LAUNCH(64, 128, 2); break;
+      case 6: TG_X3_LAUNCH(64, 64, 1); break;
+      case 7: TG_X3_LAUNCH(64, 64, 2); break;
+      default: TG_X3_LAUNCH(64, 64, 4); break;
+    }
+#undef TG_X3_LAUNCH
+    if (xp.splits > 1) add_splits(xp.splits);
+    return;
+  }
   Plan p = plan_for(d);
   GemmArgs g{d, p.kps, p.splits, 0, 0, nullptr, 0, 0};
   if (p.splits > 1) {
@@ -587,11 +757,8 @@ void gemm(const GemmDesc& d, float* work, hipStream_t st) {
     else if (bk) klaunch(k_gemm_dma<BM_, BN_, BK_, NS_, false, true, NT_, KG_>, grid, NT_, 0, st, g);     \
     else klaunch(k_gemm_dma<BM_, BN_, BK_, NS_, false, false, NT_, KG_>, grid, NT_, 0, st, g);            \
   } while (0)
-    // 128 x 128 tiles two or more per CU: a two-stage ring (64 KiB of LDS) so two blocks
-    // share a CU and one's prologue and stores overlap the other's MFMAs; the ring depth
-    // does not change the summation order
-    if (p.bm == 128 && p.bn == 128 && blocks >= 512) TG_DMA_LAUNCH(128, 128, 32, 2, 512, 1);
-    else if (p.bm == 128 && p.bn == 128) TG_DMA_LAUNCH(128, 128, 32, 3, 512, 1);
+    // (128 x 128 products of whole 32-k stages run on the split-bf16 tile)
+    if (p.bm == 128 && p.bn == 128) throw std::logic_error("gemm: a 128 x 128 f32 tile of whole stages");
     else if (p.bm == 128) TG_DMA_LAUNCH(128, 64, 32, 3, 512, 1);
     else if (p.bn == 128) TG_DMA_LAUNCH(64, 128, 32, 3, 512, 1);
     else if (p.bk == 32) TG_DMA_LAUNCH(64, 64, 32, 4, 512, 2);
@@ -636,12 +803,7 @@ void gemm(const GemmDesc& d, float* work, hipStream_t st) {
   else TG_GEMM_LAUNCH(64, 64, 64);
 #undef TG_GEMM_LAUNCH
   }
-  if (p.splits > 1) {
-    int64_t total = d.batch * d.M * d.N;
-    int64_t nb = (total + 255) / 256;
-    if (nb > 4096) nb = 4096;
-    klaunch(k_splitk_reduce, (int)nb, 256, 0, st, work, p.splits, g.sOs, d);
-  }
+  if (p.splits > 1) add_splits(p.splits);
 }
 
 // ---- products over a concatenation along k ---------------------------------------------
@@ -663,13 +825,16 @@ bool gemm_cat_ok(const GemmDesc& d, const GemmCat& c) {
   return (d.M + 127) / 128 * ((d.N + 127) / 128) < lim;
 }
 
+// The split-bf16 tile takes a second source of 16 or more k.
+static bool cat_x3(const GemmDesc& d, const GemmCat& c) { return d.M >= 128 && d.N >= 128 && d.K - c.k0 >= kXK; }
+
 static GemmArgs cat_args(const GemmDesc& d, const GemmCat& c, int64_t& blocks) {
   GemmArgs g{d, d.K, 1, 0, 0, nullptr, 0, 0};
   g.tiles_n = (int)((d.N + 127) / 128);
   g.tiles_m = (int)((d.M + 127) / 128);
   g.catA = c.a1;
   g.catAm = c.lda1;
-  g.cat_stages = (int)(c.k0 / 32);
+  g.cat_stages = (int)(c.k0 / (cat_x3(d, c) ? kXK : 32));
   blocks = (int64_t)g.tiles_n * g.tiles_m;
   return g;
 }
@@ -678,6 +843,10 @@ void gemm_cat(const GemmDesc& d, const GemmCat& c, hipStream_t st) {
   if (!gemm_cat_ok(d, c)) throw std::runtime_error("gemm_cat: unsupported operands");
   int64_t blocks = 0;
   const GemmArgs g = cat_args(d, c, blocks);
+  if (cat_x3(d, c)) {
+    klaunch(k_gemm_x3<128, 128, true, false, 1, false, true>, (unsigned)blocks, 256, 0, st, g);
+    return;
+  }
   // two or more tiles per CU: the two-stage ring (two blocks share a CU), as in gemm()
   if (blocks >= 512) klaunch(k_gemm_dma<128, 128, 32, 2, true, false, 512, 1, false, false, true, false, true>,
                              (unsigned)blocks, 512, 0, st, g);
@@ -696,6 +865,10 @@ bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, Gemm
   cfg.bkf = false;
   cfg.ns = blocks >= 512 ? 2 : 3;
   cfg.cat = true;
+  if (cat_x3(d, c)) {
+    cfg.x3 = true;
+    cfg.nt = 256;
+  }
   return true;
 }
 
@@ -704,6 +877,9 @@ bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, Gemm
 // stage st reads segment st / (K_s / BK) through its own bases. Every segment shares the
 // strides, M and N of ds[0] and its K (a multiple of the plan's k stage); one batch and
 // no split-K. The k order is segment after segment, each in the plain GEMM's order.
+
+// Segments of whole 16-k stages run on the split-bf16 tile, unsplit.
+static bool sum_x3(const GemmDesc& all, int64_t seg) { return seg % kXK == 0 && x3_ok(all); }
 
 bool gemm_sum_ok(const GemmDesc* ds, int n) {
   if (n < 2 || n > kMaxSeg) return false;
@@ -717,9 +893,10 @@ bool gemm_sum_ok(const GemmDesc* ds, int n) {
   }
   GemmDesc all = d0;
   all.K = d0.K * n;
+  if (sum_x3(all, d0.K)) return true;
   const Plan p = plan_for(all);
   if (p.splits != 1 || p.bk != 32 && p.bk != 64 || d0.K % p.bk != 0) return false;
-  if (!(p.bm == 64 && p.bn == 64) && !(p.bm == 128 && p.bn == 128)) return false;
+  if (p.bm != 64 || p.bn != 64) return false;
   const bool ak = d0.sAk == 1;
   const bool bk = d0.sBk == 1 && d0.sBn != 1;
   for (int s = 0; s < n; ++s)
@@ -731,6 +908,37 @@ void gemm_sum(const GemmDesc* ds, int n, hipStream_t st) {
   if (!gemm_sum_ok(ds, n)) throw std::runtime_error("gemm_sum: unsupported operands");
   GemmDesc all = ds[0];
   all.K = ds[0].K * n;
+  if (sum_x3(all, ds[0].K)) {
+    const int t = x3_group_tiling(&all, 1, nullptr);
+    const XTiling& x = kXTilings[t];
+    GemmArgs g{all, all.K, 1, (int)((all.N + x.bn - 1) / x.bn), (int)((all.M + x.bm - 1) / x.bm), nullptr, 0, 0};
+    g.nseg = n;
+    g.seg_stages = (int)(ds[0].K / kXK);
+    for (int s = 0; s < n; ++s) { g.segA[s] = ds[s].A; g.segB[s] = ds[s].B; }
+    const int64_t blocks = (int64_t)g.tiles_n * g.tiles_m;
+    if (blocks >= (int64_t(1) << 31)) throw std::runtime_error("gemm_sum: too many tiles");
+    const bool ak = all.sAk == 1, bk = all.sBk == 1 && all.sBn != 1;
+#define TG_X3_SEG(BM_, BN_, KG_)                                                                                      \
+  do {                                                                                                                \
+    if (ak && bk) klaunch(k_gemm_x3<BM_, BN_, true, true, KG_, true>, (unsigned)blocks, 256 * KG_, 0, st, g);         \
+    else if (ak) klaunch(k_gemm_x3<BM_, BN_, true, false, KG_, true>, (unsigned)blocks, 256 * KG_, 0, st, g);         \
+    else if (bk) klaunch(k_gemm_x3<BM_, BN_, false, true, KG_, true>, (unsigned)blocks, 256 * KG_, 0, st, g);         \
+    else klaunch(k_gemm_x3<BM_, BN_, false, false, KG_, true>, (unsigned)blocks, 256 * KG_, 0, st, g);                \
+  } while (0)
+    switch (t) {
+      case 0: TG_X3_SEG(128, 128, 1); break;
+      case 1: TG_X3_SEG(128, 128, 2); break;
+      case 2: TG_X3_SEG(128, 64, 1); break;
+      case 3: TG_X3_SEG(128, 64, 2); break;
+      case 4: TG_X3_SEG(64, 128, 1); break;
+      case 5: TG_X3_SEG(64, 128, 2); break;
+      case 6: TG_X3_SEG(64, 64, 1); break;
+      case 7: TG_X3_SEG(64, 64, 2); break;
+      default: TG_X3_SEG(64, 64, 4); break;
+    }
+#undef TG_X3_SEG
+    return;
+  }
   const Plan p = plan_for(all);
   GemmArgs g{all, all.K, 1, 0, 0, nullptr, 0, 0};
   g.tiles_n = (int)((all.N + p.bn - 1) / p.bn);
@@ -749,8 +957,7 @@ void gemm_sum(const GemmDesc* ds, int n, hipStream_t st) {
     else if (bk) klaunch(k_gemm_dma<BM_, BM_, BK_, NS_, false, true, 512, KG_, false, false, false, true>, grid, 512, 0, st, g); \
     else klaunch(k_gemm_dma<BM_, BM_, BK_, NS_, false, false, 512, KG_, false, false, false, true>, grid, 512, 0, st, g);        \
   } while (0)
-  if (p.bm == 128) TG_SEG_LAUNCH(128, 32, 3, 1);
-  else if (p.bk == 32) TG_SEG_LAUNCH(64, 32, 4, 2);
+  if (p.bk == 32) TG_SEG_LAUNCH(64, 32, 4, 2);
   else TG_SEG_LAUNCH(64, 64, 4, 2);
 #undef TG_SEG_LAUNCH
 }
@@ -765,14 +972,30 @@ int gemm_group_kind(const GemmDesc& d) {
   const Plan p{64, 64, 64, 1, d.K};
   const bool ak = d.sAk == 1;
   const bool bk = d.sBk == 1 && d.sBn != 1;
-  if (!dma_ok(d, p, ak, bk)) return -1;
-  return (ak ? 2 : 0) + (bk ? 1 : 0);
+  const int layout = (ak ? 2 : 0) + (bk ? 1 : 0);
+  SkinnyPlan sk;
+  if (x3_ok(d) && !skinny_plan(d, sk)) return 4 + layout;
+  return dma_ok(d, p, ak, bk) ? layout : -1;
 }
 
 bool gemm_prefers_group(const GemmDesc& d) {
-  if (gemm_group_kind(d) < 0) return false;
+  const int kind = gemm_group_kind(d);
+  if (kind < 0) return false;
+  if (kind >= 4) {
+    const XPlan xp = x3_plan(d);
+    return xp.splits == 1 && x3_tiles(kXTilings[xp.tiling], d) < 512;
+  }
   const Plan p = plan_for(d);
   return p.bm == 64 && p.bn == 64 && p.splits == 1;
+}
+
+// Time in us of the products' own launches, and of one grouped launch (kind >= 4), by x3_plan's figures.
+void gemm_group_times(const GemmDesc* ds, int n, double& apart, double& grouped) {
+  constexpr double kLaunch = 4.0;
+  apart = 0.0;
+  for (int q = 0; q < n; ++q) apart += kLaunch + x3_plan(ds[q]).us;
+  x3_group_tiling(ds, n, &grouped);
+  grouped += kLaunch;
 }
 
 bool gemm_epi_cfg(const GemmDesc& d, GemmEpiCfg& c, GemmArgs& g, int64_t& blocks) {
@@ -826,9 +1049,25 @@ bool gemm_epi_cfg(const GemmDesc& d, GemmEpiCfg& c, GemmArgs& g, int64_t& blocks
     c.bkf = d.sBk == 1 && d.sBn != 1;
     return blocks < (int64_t(1) << 31);
   }
-  const Plan p = plan_for(d);
   const bool ak = d.sAk == 1;
   const bool bk = d.sBk == 1 && d.sBn != 1;
+  if (x3_ok(d)) {
+    XPlan xp;
+    g = x3_args(d, nullptr, xp, blocks);
+    if (xp.splits != 1) return false;
+    const XTiling& t = kXTilings[xp.tiling];
+    c.x3 = true;
+    c.bm = t.bm;
+    c.bn = t.bn;
+    c.bk = kXK;
+    c.ns = 0;
+    c.kg = t.kg;
+    c.nt = 256 * t.kg;
+    c.ak = ak;
+    c.bkf = bk;
+    return true;
+  }
+  const Plan p = plan_for(d);
   if (p.splits != 1) return false;
   SkinnyPlan sk;
   if (!dma_ok(d, p, ak, bk) && !dma_bdw_ok(d, p, ak, bk) && use_gen_dma() && dma_gen_ok(d, ak, bk) &&
@@ -865,6 +1104,7 @@ bool gemm_epi_cfg(const GemmDesc& d, GemmEpiCfg& c, GemmArgs& g, int64_t& blocks
 
 int64_t gemm_epi_colsum_rows(const GemmEpiCfg& c, const GemmArgs& g) {
   if (c.smallk) return g.tiles_m;   // one row per block of rows
+  if (c.x3) return (int64_t)g.tiles_m * 2;   // two wavefronts along M
   // gemm_tile's wavefront grid: NW wavefronts per k group, 4 x 2 for eight with a 64-wide
   // tile, else 2 along M
   const int nw = c.nt / c.kg / 64;
@@ -872,18 +1112,21 @@ int64_t gemm_epi_colsum_rows(const GemmEpiCfg& c, const GemmArgs& g) {
   return (int64_t)g.tiles_m * wgm;
 }
 
-size_t gemm_group_table(const GemmDesc* ds, int n, std::vector<unsigned char>& image, int64_t& blocks, int& tiling) {
+size_t gemm_group_table(const GemmDesc* ds, int n, int kind, std::vector<unsigned char>& image, int64_t& blocks,
+                        int& tiling) {
   const size_t args_bytes = (size_t)n * sizeof(GemmArgs);
   const size_t starts_off = (args_bytes + 15) / 16 * 16;
   image.assign(starts_off + (size_t)(n + 1) * sizeof(uint32_t), 0);
   GemmArgs* args = reinterpret_cast<GemmArgs*>(image.data());
   uint32_t* starts = reinterpret_cast<uint32_t*>(image.data() + starts_off);
+  if (kind >= 4) tiling = x3_group_tiling(ds, n, nullptr);
+  const int bm = kind >= 4 ? kXTilings[tiling].bm : 64, bn = kind >= 4 ? kXTilings[tiling].bn : 64;
   int64_t t = 0;
   for (int q = 0; q < n; ++q) {
     const GemmDesc& d = ds[q];
     GemmArgs g{d, d.K, 1, 0, 0, nullptr, 0, 0};
-    g.tiles_n = (int)((d.N + 63) / 64);
-    g.tiles_m = (int)((d.M + 63) / 64);
+    g.tiles_n = (int)((d.N + bn - 1) / bn);
+    g.tiles_m = (int)((d.M + bm - 1) / bm);
     args[q] = g;
     starts[q] = (uint32_t)t;
     t += (int64_t)g.tiles_n * g.tiles_m * d.batch;
@@ -891,6 +1134,7 @@ size_t gemm_group_table(const GemmDesc* ds, int n, std::vector<unsigned char>& i
   starts[n] = (uint32_t)t;
   if (t >= (int64_t(1) << 31)) throw std::runtime_error("gemm group: too many tiles");
   blocks = t;
+  if (kind >= 4) return starts_off;
   // Two or more tiles per CU: 32-k stages. With every K short, the plain launch's 64 KiB
   // variant (two blocks per CU). With a long K, four wavefronts per tile and a 48 KiB
   // three-stage ring, so three blocks share a CU and overlap one another's first loads and
@@ -908,6 +1152,28 @@ void gemm_group(const void* dev_image, size_t starts_off, int n, int64_t blocks,
   const GemmArgs* table = reinterpret_cast<const GemmArgs*>(dev_image);
   const uint32_t* starts = reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(dev_image) + starts_off);
   const dim3 grid((unsigned)blocks);
+  if (kind >= 4) {
+#define TG_X3_GROUP(BM_, BN_, KG_)                                                                                    \
+  switch (kind - 4) {                                                                                                 \
+    case 3: klaunch(k_gemm_x3_group<BM_, BN_, true, true, KG_>, grid, 256 * KG_, 0, st, table, starts, n); return;    \
+    case 2: klaunch(k_gemm_x3_group<BM_, BN_, true, false, KG_>, grid, 256 * KG_, 0, st, table, starts, n); return;   \
+    case 1: klaunch(k_gemm_x3_group<BM_, BN_, false, true, KG_>, grid, 256 * KG_, 0, st, table, starts, n); return;   \
+    case 0: klaunch(k_gemm_x3_group<BM_, BN_, false, false, KG_>, grid, 256 * KG_, 0, st, table, starts, n); return;  \
+    default: throw std::runtime_error("gemm group: bad kind");                                                        \
+  }
+    switch (tiling) {
+      case 0: TG_X3_GROUP(128, 128, 1)
+      case 1: TG_X3_GROUP(128, 128, 2)
+      case 2: TG_X3_GROUP(128, 64, 1)
+      case 3: TG_X3_GROUP(128, 64, 2)
+      case 4: TG_X3_GROUP(64, 128, 1)
+      case 5: TG_X3_GROUP(64, 128, 2)
+      case 6: TG_X3_GROUP(64, 64, 1)
+      case 7: TG_X3_GROUP(64, 64, 2)
+      default: TG_X3_GROUP(64, 64, 4)
+    }
+#undef TG_X3_GROUP
+  }
   if (tiling == 2) {   // 32-k stages on four wavefronts, 48 KiB: three blocks per CU
     switch (kind) {
       case 3: klaunch(k_gemm_dma_group<64, 64, 32, 3, true, true, 256, 1>, grid, 256, 0, st, table, starts, n); return;

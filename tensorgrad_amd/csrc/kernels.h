@@ -301,12 +301,12 @@ void attention_bwd(const AttnBwdDesc& a, hipStream_t st);
 // `work` must hold gemm_workspace_floats(d) floats (split-K partials).
 int64_t gemm_workspace_floats(const GemmDesc& d);
 void gemm(const GemmDesc& d, float* work, hipStream_t st);
-// Grouped launch of independent GEMMs (whole-K 64 x 64 tiles, no split-K). Problems of one
-// launch share a kind: gemm_group_kind(d) is 0..3, or -1 when d cannot run grouped.
-// gemm_group_table fills the device image of the problem table (returns the offset of
+// Grouped launch of independent GEMMs (no split-K). Problems of one launch share a kind:
+// gemm_group_kind(d) is 4..7 on the split-bf16 tile, 0..3 on 64 x 64 f32 tiles, or -1 when d
+// cannot run grouped. gemm_group_table fills the device image of the problem table (returns the offset of
 // its tile-start array, sets the launch's block count and the tiling gemm_group takes:
-// 1 for 32-k stages, two blocks per CU, when the launch has two or more tiles per CU and
-// short K, else 0); the image must be copied to device memory and stay there while the
+// an entry of the split tile's table (kinds 4..7); 1 for 32-k stages, two blocks per CU,
+// when the launch has two or more f32 tiles per CU and short K, else 0); the image must be copied to device memory and stay there while the
 // launch can run.
 int gemm_group_kind(const GemmDesc& d);
 // A GEMM whose epilogue runs a fused element group (a kernel generated at run time): the
@@ -328,6 +328,7 @@ struct GemmEpiCfg {
   bool smallk = false;    // the small-K kernel (smallk_tile, bm rows of k padded to bk) instead of the tile
   bool gen = false;       // the element-wise tile (both operands one element per lane, partial k stages)
   bool tiny = false;      // the tiny kernel (tiny_tile, bm lanes per output; no column partials)
+  bool x3 = false;        // the split-bf16 tile (x3_tile; kg groups of 256 threads)
   bool skinny = false;    // the skinny kernel (skinny_tile, bm column tiles, bk: 16-byte A loads; no column partials)
 };
 // Rows of the f64 column partials an epilogue with colsum_out writes for this launch
@@ -344,10 +345,13 @@ struct GemmCat {
 bool gemm_cat_ok(const GemmDesc& d, const GemmCat& c);
 void gemm_cat(const GemmDesc& d, const GemmCat& c, hipStream_t st);
 bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, gd::GemmArgs& g, int64_t& blocks);
-// True when d on its own would run one pass of 64 x 64 tiles (the grouped tiling); the
-// grouped launch's k-stage depth follows its own tile count, as a plain launch's does.
+// True when d on its own would run one pass of tiles that does not fill the chip twice; the
+// grouped launch's tiling (on f32 tiles: its k-stage depth) follows its own tile count.
 bool gemm_prefers_group(const GemmDesc& d);
-size_t gemm_group_table(const GemmDesc* ds, int n, std::vector<unsigned char>& image, int64_t& blocks, int& tiling);
+// Estimated times (us) of products of one kind >= 4 in launches of their own and in one.
+void gemm_group_times(const GemmDesc* ds, int n, double& apart, double& grouped);
+size_t gemm_group_table(const GemmDesc* ds, int n, int kind, std::vector<unsigned char>& image, int64_t& blocks,
+                        int& tiling);
 void gemm_group(const void* dev_image, size_t starts_off, int n, int64_t blocks, int kind, int tiling,
                 hipStream_t st);
 

@@ -3113,23 +3113,33 @@ bool Runtime::only_optimizer_reads(int t) const {
 void Runtime::plan_gemm_groups() {
   defer_gemm_.assign(ops_.size(), 0);
   if (!use_gemm_group_) return;
-  std::vector<int> cand[4];
+  std::vector<int> cand[8];
+  std::vector<tgk::GemmDesc> descs[8];
   int64_t tiles[4] = {0, 0, 0, 0};
   for (size_t i = 0; i < ops_.size(); ++i) {
     if ((kinds_[i] != "matmul" && kinds_[i] != "matmul_batched") || virtual_[i]) continue;
     const int a = fld((int)i, "a"), b = fld((int)i, "b");
     if (kinds_[T_[view_[a].root].src] == "one_hot" || kinds_[T_[view_[b].root].src] == "one_hot") continue;
     tgk::GemmDesc d{};
-    if (!gemm_desc((int)i, d) || tgk::gemm_workspace_floats(d) <= 0) continue;
-    if (!only_optimizer_reads(O((int)i).at("out").i32())) continue;
+    if (!gemm_desc((int)i, d)) continue;
     const int kind = tgk::gemm_group_kind(d);
-    if (kind < 0) continue;
+    if (kind < 0 || (tgk::gemm_workspace_floats(d) <= 0 && !(kind >= 4 && tgk::gemm_prefers_group(d)))) continue;
+    if (!only_optimizer_reads(O((int)i).at("out").i32())) continue;
     cand[kind].push_back((int)i);
-    tiles[kind] += ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
+    descs[kind].push_back(d);
+    if (kind < 4) tiles[kind] += ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
   }
-  for (int k = 0; k < 4; ++k)
-    if (tiles[k] >= 256)
+  for (int k = 0; k < 8; ++k) {
+    if (cand[k].size() < 2) continue;
+    bool defer = k < 4 && tiles[k] >= 256;
+    if (k >= 4) {
+      double apart = 0.0, grouped = 0.0;
+      tgk::gemm_group_times(descs[k].data(), (int)descs[k].size(), apart, grouped);
+      defer = grouped < apart;
+    }
+    if (defer)
       for (int i : cand[k]) defer_gemm_[i] = 1;
+  }
 }
 
 int Runtime::epi_group(int op, int out, const tgk::GemmDesc& d, bool& store_c, const CatFwd* cat) const {
@@ -3522,7 +3532,7 @@ void Runtime::emit_gemm_group(const std::vector<DeferredGemm>& grp) {
     std::vector<unsigned char> img;
     int64_t blocks = 0;
     int tiling = 0;
-    const size_t off = tgk::gemm_group_table(ds.data(), (int)ds.size(), img, blocks, tiling);
+    const size_t off = tgk::gemm_group_table(ds.data(), (int)ds.size(), kind, img, blocks, tiling);
     if (plan_only_) return [](hipStream_t) {};
     void* dev = nullptr;
     hip_check(hipMalloc(&dev, img.size()), "hipMalloc(gemm group table)");
@@ -3535,7 +3545,7 @@ void Runtime::emit_gemm_group(const std::vector<DeferredGemm>& grp) {
 }
 
 void Runtime::flush_deferred_gemms() {
-  for (int kind = 0; kind < 4; ++kind) {
+  for (int kind = 0; kind < 8; ++kind) {
     std::vector<DeferredGemm> grp;
     for (const DeferredGemm& g : deferred_gemms_)
       if (g.kind == kind) grp.push_back(g);

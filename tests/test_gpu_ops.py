@@ -653,6 +653,108 @@ def test_matmul(case):
     gemm_close(got, want)
 
 
+# [M, K] x [K, N] on the split-bf16 tile: tile edges and one past them, the smallest product it takes, k of one whole
+# stage more or less, every tiling (few tiles by four groups, 128-wide ones), split K, a batch with strided views
+X3 = [(64, 64, 32), (65, 64, 33), (127, 129, 47), (128, 128, 48), (129, 191, 63), (191, 127, 65), (64, 300, 95),
+      (1000, 64, 257), (300, 5003, 64), (128, 64, 1024), (130, 70, 1100), (256, 256, 9000), (4100, 260, 81),
+      (2048, 2050, 130)]
+
+
+def _product(M, N, K, ta, tb):
+    def body():
+        a = tensor_input('a', [K, M] if ta else [M, K])
+        b = tensor_input('b', [N, K] if tb else [K, N])
+        return O.matmul(O.swap_axes(a, -1, -2) if ta else a, O.swap_axes(b, -1, -2) if tb else b)
+    return body
+
+
+@pytest.mark.parametrize('ta,tb', [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize('M,N,K', X3)
+def test_matmul_split_tile(M, N, K, ta, tb):
+    """f32 products on bf16 matrix cores against the oracle's f64 sums. Tolerance: every running-sum addition (one per
+    32 k) and every MFMA of a 32-k part rounds by at most 2^-24 of the sum it makes, with signs that do not line up."""
+    a, b = _rand([K, M] if ta else [M, K], 141), _rand([N, K] if tb else [K, N], 142)
+    got, want = run_both(_product(M, N, K, ta, tb), {'a': a, 'b': b})
+    gemm_close(got, want, 2.0 ** -24 * (4 + (K / 16) ** 0.5))
+
+
+def test_matmul_split_tile_wide_values():
+    """Values over 60 orders of magnitude (rows and columns scaled by powers of two): each output is as close to its f64
+    value, relative to the sum of its terms' magnitudes, as one of ordinary size; zeros and single ones stay exact."""
+    M, N, K = 200, 130, 300
+    a, b = _rand([M, K], 143), _rand([K, N], 144)
+    a *= (2.0 ** np.linspace(-60, 60, M)).astype(np.float32)[:, None]
+    b *= (2.0 ** np.linspace(40, -40, N)).astype(np.float32)[None, :]
+    b[:, 7] = 0
+    b[:, 9] = np.eye(K, dtype=np.float32)[5]
+    got, want = run_both(_product(M, N, K, False, False), {'a': a, 'b': b})
+    terms = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert np.all(np.abs(got - want.astype(np.float64)) <= 2.0 ** -22 * terms)
+    assert np.all(got[:, 7] == 0) and np.array_equal(got[:, 9], a[:, 5])
+
+
+@pytest.mark.parametrize('M,N,K', [(130, 70, 40), (300, 256, 300), (256, 256, 2050)])
+def test_matmul_split_tile_infinities(M, N, K):
+    """Infinities, NaN and values that round to infinity in bf16 give what f32 products give, and leave the other rows
+    and columns alone."""
+    a, b = _rand([M, K], 145), _rand([K, N], 146)
+    a[3, 5], a[70, K - 1], a[9, 0], b[2, 11] = np.inf, -np.inf, np.nan, np.inf
+    a[20] = 0
+    a[20, 1], b[1] = 3.4e38, np.float32(1e-3) * b[1]
+    got, want = run_both(_product(M, N, K, False, False), {'a': a, 'b': b})
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(got)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    row = np.arange(M) != 20
+    keep = ok & row[:, None]
+    gemm_close(got[keep], want[keep])
+    gemm_close(got[20][ok[20]], want[20][ok[20]])
+
+
+def test_matmul_split_tile_batched_and_summed():
+    """Batched head views (two batch strides), and a sum of products whose segments hold an infinity."""
+    B, T, H, d = 3, 100, 2, 80
+    x, y = _rand([B, T, H * d], 147), _rand([B, T, H * d], 148)
+
+    def scores():
+        q, k = (O.split_heads(tensor_input(n, [B, T, H * d]), H) for n in 'xy')
+        return O.matmul(q, O.swap_axes(k, -1, -2))
+    got, want = run_both(scores, {'x': x, 'y': y})
+    gemm_close(got, want)
+
+    M, N, K = 192, 70, 48
+    ins = {f'a{q}': _rand([M, K], 150 + q) for q in range(3)}
+    ins.update({f'b{q}': _rand([N, K], 160 + q) for q in range(3)})
+
+    def total():
+        ps = [O.matmul(tensor_input(f'a{q}', [M, K]), O.swap_axes(tensor_input(f'b{q}', [N, K]), -1, -2)) for q in range(3)]
+        return O.relu(O.add(O.add(ps[0], ps[1]), ps[2]))
+    for inf in (False, True):
+        if inf:
+            ins['a1'][100, 20] = np.inf
+        got, want = run_both(total, ins)
+        assert np.array_equal(np.isinf(got), np.isinf(want)) and not np.isnan(got).any()
+        ok = np.isfinite(want)
+        gemm_close(got[ok], want[ok])
+
+
+@pytest.mark.parametrize('M,k0,k1,N', [(128, 32, 16, 128), (300, 64, 17, 130), (2000, 32, 63, 256), (129, 96, 32, 200)])
+def test_concat_product_split_tile(M, k0, k1, N):
+    """A product over two sources with 16 or more k in the second, whole and with an infinity in each source."""
+    ins = {'s0': _rand([M, k0], 171), 's1': _rand([M, k1], 172), 'w': _rand([k0 + k1, N], 173)}
+
+    def body():
+        return O.matmul(O.concat([tensor_input('s0', [M, k0]), tensor_input('s1', [M, k1])], -1),
+                        tensor_input('w', [k0 + k1, N]))
+    for inf in (False, True):
+        if inf:
+            ins['s0'][5, 3] = ins['s1'][100, k1 - 1] = np.inf
+        got, want = run_both(body, ins)
+        assert np.array_equal(np.isinf(got), np.isinf(want)) and not np.isnan(got).any()
+        ok = np.isfinite(want)
+        gemm_close(got[ok], want[ok])
+
+
 @pytest.mark.parametrize('sa,sb,ta', [([256, 1], [1, 64], False), ([256, 64], [64, 1], False),
                                       ([1, 256], [256, 64], False), ([64, 4096], [4096, 1], False),
                                       ([3, 1], [1, 5], False), ([256, 1], [64, 1], True),
