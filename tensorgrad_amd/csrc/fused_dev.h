@@ -110,6 +110,20 @@ __device__ __forceinline__ double wave_allsum(double v) { return wave_allreduce(
 __device__ __forceinline__ float wave_allsum(float v) { return wave_allreduce(v, WaveAdd()); }
 __device__ __forceinline__ float wave_allmax(float v) { return wave_allreduce(v, WaveMax()); }
 
+// The same over a block of up to 16 wavefronts: their results in order through `red` (one double each), which is free
+// again when every thread has passed the second barrier.
+template <class T, class Op> __device__ __forceinline__ T block_allreduce(T v, double* red, Op op) {
+  v = wave_allreduce(v, op);
+  if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = (double)v;
+  __syncthreads();
+  T t = (T)red[0];
+  for (unsigned w = 1; w < blockDim.x / 64; ++w) t = op(t, (T)red[w]);
+  __syncthreads();
+  return t;
+}
+__device__ __forceinline__ double block_allsum(double v, double* red) { return block_allreduce(v, red, WaveAdd()); }
+__device__ __forceinline__ float block_allmax(float v, double* red) { return block_allreduce(v, red, WaveMax()); }
+
 __device__ __forceinline__ double js_max(double a, double b) {
   if (isnan(a) || isnan(b)) return __longlong_as_double(0x7ff8000000000000LL);
   if (a == 0.0 && b == 0.0) return (signbit(a) && signbit(b)) ? -0.0 : 0.0;

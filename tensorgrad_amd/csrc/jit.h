@@ -18,13 +18,17 @@ namespace tgk {
 struct JitKernel {
   std::string name;   // tg_<hash of body>
   std::string body;   // extern "C" __global__ definition
-  int64_t grid = 0;   // blocks of 256 threads
+  int64_t grid = 0;   // blocks
+  int threads = 256;  // of a block
   bool gemm = false;  // a GEMM with a fused epilogue (its program needs gemm_dev.h)
 };
 
 // Source of a GEMM kernel (gemm_dev.h's tile) whose epilogue runs the element program p
 // (one element per call, vec = 1) on each product element instead of storing it.
 JitKernel gemm_epi_kernel(const FusedProgram& p, const FusedInstr* code, const GemmEpiCfg& c);
+
+// Widest row of a row group: one wavefront's, and (several rows, generated kernels only) one block's.
+constexpr int64_t kWaveRow = 1024, kBlockRow = 16384;
 
 // Source of the kernel for `p` (its code[] instructions) over n threads' runs (element
 // form: elements / vec) or n rows (row form).

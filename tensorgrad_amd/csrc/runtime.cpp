@@ -2052,9 +2052,9 @@ void Runtime::form_groups() {
     if (red) {
       const int a = fld((int)i, "a");
       In = T_[a].shape;
-      // Rows up to 1024 wide; a single row (a whole-tensor sum) up to kWideRow in generated
-      // kernels. Wider rows run as standalone reductions.
-      const int64_t maxd = use_jit_ && T_[a].numel == In.back() ? kWideRow : 1024;
+      // Rows up to 1024 wide, a wavefront each; in generated kernels also a single row (a whole-tensor sum) up to
+      // kWideRow and several rows up to kBlockRow, a block each. Wider rows run as standalone reductions.
+      const int64_t maxd = !use_jit_ ? tgk::kWaveRow : T_[a].numel == In.back() ? kWideRow : tgk::kBlockRow;
       if (In.empty() || In.back() < 1 || In.back() > maxd || T_[a].numel <= 0) continue;
     }
     std::vector<int> cands;
@@ -2480,6 +2480,7 @@ void Runtime::lower_group(int gi) {
     JitSlot& sl = jit_slots_.back();
     sl.name = jk.name;
     sl.grid = jk.grid;
+    sl.threads = jk.threads;
     for (int k = 0; k < p.n_in; ++k) sl.args.in[k] = p.in[k];
     for (int k = 0; k < p.n_out; ++k) sl.args.out[k] = p.out[k];
     sl.args.seed = p.seed;

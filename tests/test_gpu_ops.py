@@ -278,6 +278,36 @@ def test_softmaxes_and_causal_mask():
 
 
 CE_SHAPES = [(64, 27), (128, 10), (50, 65), (7, 130), (4096, 65)]
+# rows of a block each: one past a wavefront's, one chunk more or less, 256 / 512 / 1024 threads, the widest
+WIDE_ROWS = [(3, 1025), (2, 2048), (5, 4096), (3, 4097), (40, 5003), (2, 8193), (2, 16384)]
+
+
+@pytest.mark.parametrize('R,D', WIDE_ROWS)
+def test_row_groups_of_wide_rows(R, D):
+    """Rows of up to 16384 run as row groups of a block each: a log-softmax with its one-hot pick and gradient chain, a
+    row mean read back by every column, dropout; f64 row sums in another order than the evaluator's, so at most one f32
+    ulp apart (the log-softmax subtracts two such values: the ulp of its largest term)."""
+    x, b = _rand([R, D], 61, -6, 6), _rand([D], 62)
+    t = np.random.default_rng(63).integers(0, D, size=[R]).astype(np.int32)
+    ins = {'x': x, 'b': b, 't': t}
+
+    def lsm():
+        return O.log_softmax(O.add(tensor_input('x', [R, D]), tensor_input('b', [D])))
+    got, want = run_both(lsm, ins)
+    assert np.max(np.abs(got - want.astype(np.float64))) <= np.spacing(np.float32(np.max(np.abs(want))))
+
+    def grad():
+        oh = O.one_hot(tensor_input('t', [R], 'i32'), D, 'f32')
+        x = tensor_input('x', [R, D])
+        s = O.reshape(O.sum_(O.mul(x, oh), -1), [R, 1])
+        return O.dropout(O.sub(O.mul(oh, 0.25), O.mul(O.broadcast_to(s, [R, D]), O.mean(x, -1, keep_dims=True))), 0.1)
+    got, want = run_both(grad, ins)
+    near(got, want, 2)   # the mean's ulp, carried through a product that rounds again
+    g = trace_fn(lsm)
+    assert 'rowfused' in _run_native(g, ins)[1] and 'softmax' not in _run_native(g, ins)[1]
+    got, want = run_both(lambda: nn.cross_entropy(O.add(tensor_input('x', [R, D]), tensor_input('b', [D])),
+                                                  tensor_input('t', [R], 'i32')), ins)
+    near(got, want)
 
 
 @pytest.mark.parametrize('R,D', CE_SHAPES)
