@@ -1407,9 +1407,12 @@ __global__ void k_segment_finish(const double* __restrict__ part, int64_t N, int
   }
 }
 
-// Small vocabularies (V * rows <= kScatterScanMax) need no sort: block (v, column chunk)
-// of four wavefronts runs scatter_scan_block (scatter_dev.h). One launch, no workspace.
+// Small vocabularies (V * rows <= kScatterScanMax), and larger ones over few rows, need no
+// sort: block (v, column chunk) of four wavefronts runs scatter_scan_block (scatter_dev.h).
+// One launch, no workspace. With few rows the sort's one block and its three launches cost
+// more than every token's block reading all the row ids (from L2).
 constexpr int64_t kScatterScanMax = int64_t(1) << 22;
+constexpr int64_t kScatterFewRows = 8192, kScatterScanFew = int64_t(1) << 26;
 
 __global__ __launch_bounds__(256) void k_scatter_scan(const int32_t* __restrict__ idx, int64_t rows,
                                                       const float* __restrict__ dy, int64_t N,
@@ -1418,7 +1421,9 @@ __global__ __launch_bounds__(256) void k_scatter_scan(const int32_t* __restrict_
   scatter_scan_block<4>(idx, rows, dy, N, out, (int)blockIdx.x, blockIdx.y * 256ll, L);
 }
 
-inline bool scatter_scans(int64_t rows, int64_t V) { return V * rows <= kScatterScanMax; }
+inline bool scatter_scans(int64_t rows, int64_t V) {
+  return V * rows <= (rows <= kScatterFewRows ? kScatterScanFew : kScatterScanMax);
+}
 
 inline int grid_for(int64_t n) {
   int64_t b = (n + 255) / 256;

@@ -826,6 +826,8 @@ def test_matmul_batched_head_views():
     (50, 300, 20000, False),   # too many rows for the LDS stash; N > 256 columns
     (7, 33, 5000, True),       # one token owns most rows: long buckets cut into many items
     (2, 8, 64, False),
+    (8000, 40, 8192, False),   # few rows: every token's block scans them all
+    (2000, 24, 8193, False),   # one row more: sorted
 ])
 def test_embedding_gather_and_scatter(V, N, rows, skew):
     rng = np.random.default_rng(18)
