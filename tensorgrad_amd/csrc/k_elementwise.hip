@@ -9,6 +9,8 @@
 // for 256 CUs so that large tensors are covered by resident waves.
 #include "kernels.h"
 
+#include <algorithm>
+
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
@@ -248,6 +250,13 @@ __global__ __launch_bounds__(256) void k_concat_last(uint32_t* __restrict__ dst,
   }
 }
 
+// `quads` 16-byte units, then `words` single ones.
+__global__ void k_copy_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, int64_t quads, int64_t words) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = t; i < quads; i += step) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+  for (int64_t i = t; i < words; i += step) dst[quads * 4 + i] = src[quads * 4 + i];
+}
+
 __global__ void k_fill(uint32_t* __restrict__ dst, uint32_t bits, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     dst[i] = bits;
@@ -420,6 +429,14 @@ void strided_copy(void* dst, const void* src, const Strided& sp, int64_t n, hipS
   if (b > 16384) b = 16384;
   if (vec == 4) klaunch(k_copy32<4>, (int)b, 256, 0, st, (uint32_t*)dst, (const uint32_t*)src, c, (uint32_t)nv);
   else klaunch(k_copy32<1>, (int)b, 256, 0, st, (uint32_t*)dst, (const uint32_t*)src, c, (uint32_t)nv);
+}
+
+void copy_words(void* dst, const void* src, int64_t bytes, hipStream_t st) {
+  if (bytes <= 0) return;
+  const bool al = (((uintptr_t)dst | (uintptr_t)src) & 15) == 0;
+  const int64_t quads = al ? bytes / 16 : 0, words = (bytes - quads * 16) / 4;
+  const int64_t b = (std::max(quads, words) + kThreads - 1) / kThreads;
+  klaunch(k_copy_words, (int)std::min<int64_t>(b, 4096), kThreads, 0, st, (uint32_t*)dst, (const uint32_t*)src, quads, words);
 }
 
 void fill(void* dst, int dt, double value, int64_t n, hipStream_t st) {

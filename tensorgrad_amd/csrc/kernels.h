@@ -97,6 +97,8 @@ struct ConcatLast {
 };
 void concat_last(uint32_t* dst, const ConcatLast& c, int64_t rows, hipStream_t st);
 void fill(void* dst, int dt, double value, int64_t n, hipStream_t st);
+// bytes (a multiple of 4) from src to dst, either of them device memory or pinned host memory, by a kernel.
+void copy_words(void* dst, const void* src, int64_t bytes, hipStream_t st);
 void arange(void* dst, int dt, int64_t n, hipStream_t st);
 void one_hot(const int32_t* idx, int64_t rows, int64_t depth, void* out, int dt, hipStream_t st);
 // Stochastic ops: the seed lives in device memory (a per-step tensor input).

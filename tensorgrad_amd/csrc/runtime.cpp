@@ -313,8 +313,9 @@ class Runtime {
   const void* dev_table(const std::string& key, const void* data, size_t bytes);
   std::vector<int> state_roots_;
 
-  hipGraph_t graph_ = nullptr;
-  hipGraphExec_t graph_exec_ = nullptr;
+  // the captured step: [0] user inputs already in the input region, [1] fetched from pinned host memory
+  hipGraph_t graph_[2] = {nullptr, nullptr};
+  hipGraphExec_t graph_exec_[2] = {nullptr, nullptr};
   bool plan_only_ = false;
 
   // Element-wise fusion groups: members in op order; the group runs at its first op.
@@ -463,13 +464,13 @@ class Runtime {
   void launch_all(hipStream_t st);
   void upload_inputs(int n, const char* const* names, const void* const* data, const int64_t* nbytes, bool device);
   void advance_scalars(bool optimizer);
-  void upload_scalars();
+  void launch_step(hipStream_t st, bool host);
  public:
   void stage_batch(int slot, int n, const char* const* names, const void* const* data, const int64_t* nbytes);
   float step_staged(int slot);
  private:
-  void ensure_graph();
-  void replay();
+  void ensure_graph(bool host);
+  void replay(bool host);
   float* cur_ws_ = nullptr;            // workspace of the node being bound
   unsigned* cur_counters_ = nullptr;   // launch-completion counters of the node being bound
   // Scratch-only step (tg_step_noalloc): the launches again, with every node that uses the
@@ -671,8 +672,8 @@ void Runtime::read_document() {
 }
 
 Runtime::~Runtime() {
-  if (graph_exec_) hipGraphExecDestroy(graph_exec_);
-  if (graph_) hipGraphDestroy(graph_);
+  for (hipGraphExec_t g : graph_exec_) if (g) hipGraphExecDestroy(g);
+  for (hipGraph_t g : graph_) if (g) hipGraphDestroy(g);
   if (stream_) { hipStreamSynchronize(stream_); hipStreamDestroy(stream_); }
   if (arena_) hipFree(arena_);
   if (input_region_) hipFree(input_region_);
@@ -4563,11 +4564,12 @@ float Runtime::step_noalloc(int n, const char* const* names, const void* const* 
   std::lock_guard<std::mutex> g(g_noalloc_mu);
   advance_scalars(true);
   upload_inputs(n, names, data, nbytes, true);
+  tgk::copy_words(input_region_ + user_bytes_, staging_ + user_bytes_, (int64_t)(input_region_bytes_ - user_bytes_), stream_);
   // The counters must start at zero; the scratch keeps whatever the last call left.
   if (counter_slots_) tgk::fill(noalloc_counters_, tgk::DT_I32, 0.0, counter_slots_, stream_);
   for (auto& f : noalloc_launch_) f(stream_);
   apply_copy_writebacks(stream_);
-  hip_check(hipMemcpyAsync(loss_host_, dptr(outputs_.at(0)), 4, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync(D2H)");
+  tgk::copy_words(loss_host_, dptr(outputs_.at(0)), 4, stream_);
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   return loss_host_[0];
 }
@@ -4597,32 +4599,48 @@ void Runtime::apply_copy_writebacks(hipStream_t st) {
   }
 }
 
-// One execution of the step: a replay of the captured graph, or (graphs disabled) the
-// same launches issued directly on the stream.
-void Runtime::replay() {
-  if (!use_graph_) {
-    launch_all(stream_);
-    apply_copy_writebacks(stream_);
-    return;
-  }
-  ensure_graph();
-  hip_check(hipGraphLaunch(graph_exec_, stream_), "hipGraphLaunch");
+// One step's launches. The per-step scalars come from pinned host memory by the step's first kernel, with `host` the user
+// inputs too (they precede them there), and the loss goes to pinned host memory by its last: a copy of a few bytes each
+// way cost the stream about 8 us a step, a kernel node of the captured step about 2.
+void Runtime::launch_step(hipStream_t st, bool host) {
+  const size_t from = host ? 0 : user_bytes_;
+  tgk::copy_words(input_region_ + from, staging_ + from, (int64_t)(input_region_bytes_ - from), st);
+  launch_all(st);
+  apply_copy_writebacks(st);
+  if (opt_cfg_) tgk::copy_words(loss_host_, dptr(outputs_.at(0)), 4, st);
 }
 
-void Runtime::ensure_graph() {
-  if (graph_exec_) return;
+// User inputs above this size go from pinned host memory by the copy engine, before the step.
+static constexpr size_t kFetchBytes = 1 << 20;
+
+// One execution of the step: a replay of the captured graph (one per way the inputs come, captured at its first use), or
+// (graphs disabled) the same launches issued directly on the stream.
+void Runtime::replay(bool host) {
+  if (host && user_bytes_ > kFetchBytes) {
+    hip_check(hipMemcpyAsync(input_region_, staging_, user_bytes_, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(H2D)");
+    host = false;
+  }
+  if (!use_graph_) {
+    launch_step(stream_, host);
+    return;
+  }
+  ensure_graph(host);
+  hip_check(hipGraphLaunch(graph_exec_[host], stream_), "hipGraphLaunch");
+}
+
+void Runtime::ensure_graph(bool host) {
+  if (graph_exec_[host]) return;
   hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   try {
-    launch_all(stream_);
-    apply_copy_writebacks(stream_);
+    launch_step(stream_, host);
   } catch (...) {
     hipGraph_t g;
     hipStreamEndCapture(stream_, &g);
     if (g) hipGraphDestroy(g);
     throw;
   }
-  hip_check(hipStreamEndCapture(stream_, &graph_), "hipStreamEndCapture");
-  hip_check(hipGraphInstantiate(&graph_exec_, graph_, nullptr, nullptr, 0), "hipGraphInstantiate");
+  hip_check(hipStreamEndCapture(stream_, &graph_[host]), "hipStreamEndCapture");
+  hip_check(hipGraphInstantiate(&graph_exec_[host], graph_[host], nullptr, nullptr, 0), "hipGraphInstantiate");
 }
 
 void Runtime::advance_scalars(bool optimizer) {
@@ -4653,12 +4671,6 @@ void Runtime::advance_scalars(bool optimizer) {
   }
 }
 
-void Runtime::upload_scalars() {
-  if (input_region_bytes_ > user_bytes_)
-    hip_check(hipMemcpyAsync(input_region_ + user_bytes_, staging_ + user_bytes_, input_region_bytes_ - user_bytes_,
-                             hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(H2D scalars)");
-}
-
 void Runtime::upload_inputs(int n, const char* const* names, const void* const* data, const int64_t* nbytes,
                             bool device) {
   // Validate the whole record before touching any state.
@@ -4684,9 +4696,6 @@ void Runtime::upload_inputs(int n, const char* const* names, const void* const* 
     else
       memcpy(staging_ + input_offset_[t], data[i], (size_t)nbytes[i]);
   }
-  if (!device && user_bytes_)
-    hip_check(hipMemcpyAsync(input_region_, staging_, user_bytes_, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync(H2D)");
-  upload_scalars();
 }
 
 // Device-resident batches for measurement and for callers that prefetch: slot k holds a
@@ -4716,11 +4725,8 @@ float Runtime::step_staged(int slot) {
   if (!opt_cfg_) throw Error(TG_INVALID_ARGUMENT, "step: graph has no optimizer (use run)");
   advance_scalars(true);
   if (slot < 0 || slot >= (int)slots_.size() || !slots_[slot]) throw Error(TG_INVALID_ARGUMENT, "step: slot not staged");
-  if (user_bytes_)
-    hip_check(hipMemcpyAsync(input_region_, slots_[slot], user_bytes_, hipMemcpyDeviceToDevice, stream_), "hipMemcpyAsync(D2D)");
-  upload_scalars();
-  replay();
-  hip_check(hipMemcpyAsync(loss_host_, dptr(outputs_.at(0)), 4, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync(D2H)");
+  if (user_bytes_) tgk::copy_words(input_region_, slots_[slot], (int64_t)user_bytes_, stream_);
+  replay(false);
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   return loss_host_[0];
 }
@@ -4729,9 +4735,7 @@ float Runtime::step(int n, const char* const* names, const void* const* data, co
   if (!opt_cfg_) throw Error(TG_INVALID_ARGUMENT, "step: graph has no optimizer (use run)");
   advance_scalars(true);
   upload_inputs(n, names, data, nbytes, device);
-  replay();
-  int lt = outputs_.at(0);
-  hip_check(hipMemcpyAsync(loss_host_, dptr(lt), 4, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync(D2H)");
+  replay(!device);
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   return loss_host_[0];
 }
@@ -4746,7 +4750,7 @@ void Runtime::run(int n, const char* const* names, const void* const* data, cons
     throw Error(TG_INVALID_ARGUMENT, "tensorgrad: missing input '" + opt_cfg_->at(f).str() + "'");
   }
   upload_inputs(n, names, data, nbytes, false);
-  replay();
+  replay(true);
   int o = outputs_.at(0);
   if (out_bytes != T_[o].numel * 4) throw Error(TG_INVALID_ARGUMENT, "run: output buffer has the wrong size");
   if (!view_[o].contiguous()) throw Error(TG_INTERNAL, "run: output is not contiguous");
@@ -4914,12 +4918,12 @@ double Runtime::time_kinds(const std::string& kinds, int iters, int* launches) {
 }
 
 double Runtime::time_replays(int steps) {
-  if (use_graph_) ensure_graph();
+  if (use_graph_) ensure_graph(false);
   hipEvent_t a, b;
   hip_check(hipEventCreate(&a), "hipEventCreate");
   hip_check(hipEventCreate(&b), "hipEventCreate");
   hip_check(hipEventRecord(a, stream_), "hipEventRecord");
-  for (int i = 0; i < steps; ++i) replay();
+  for (int i = 0; i < steps; ++i) replay(false);
   hip_check(hipEventRecord(b, stream_), "hipEventRecord");
   hip_check(hipEventSynchronize(b), "hipEventSynchronize");
   float ms = 0;
