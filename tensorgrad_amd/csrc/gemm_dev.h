@@ -537,8 +537,8 @@ struct StoreC {   // (tile_finish stores it)
 // The bf16 MFMAs run at 16 times the f32 rate. An f32 value is exactly the sum of three bf16 values (round to nearest,
 // then the same of what is left, twice: 8 + 8 + 8 bits), so a product is nine bf16 products, of which the three below
 // 2^-25 of the largest (mid * low, low * mid, low * low) are left out: six MFMAs in place of sixteen's worth of time.
-// Accuracy against 64 bits is no worse than the f32 tile's (norm-wise, K = 256 .. 4096: 0.9e-7 .. 2.3e-7 against
-// 1.2e-7 .. 2.3e-7): the products are exact, an MFMA adds 16 of them with one rounding where the f32 one adds two, and
+// Accuracy against 64 bits is no worse than the f32 tile's (norm-wise, K = 512 .. 4096: 0.9e-7 .. 1.3e-7 against
+// 1.1e-7 .. 1.8e-7): the products are exact, an MFMA adds 16 of them with one rounding where the f32 one adds two, and
 // every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum.
 // Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
 // are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile.
@@ -631,7 +631,8 @@ struct XTile {
     if (n == 2) *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
     else *reinterpret_cast<uint32_t*>(p) = v[0];
   }
-  __device__ __forceinline__ static void store(const float* q, char* L, int tid) {
+  template <bool SIGNED>   // SIGNED: times sign (1 or -1)
+  __device__ __forceinline__ static void store(const float* q, char* L, int tid, float sign) {
     constexpr int W = KFAST ? 2 : PK / 2;          // pairs of k in a unit
     constexpr int UNITS = KFAST ? PER / 4 : 2;
 #pragma unroll
@@ -640,7 +641,10 @@ struct XTile {
       const int k = KFAST ? (tid & 3) * 4 : (tid / (ROWS / 2)) * PK;
       uint32_t h[W], m[W], l[W];
 #pragma unroll
-      for (int u = 0; u < W; ++u) split3(q[(e * W + u) * 2], q[(e * W + u) * 2 + 1], h[u], m[u], l[u]);
+      for (int u = 0; u < W; ++u) {
+        const float x0 = q[(e * W + u) * 2], x1 = q[(e * W + u) * 2 + 1];
+        split3(SIGNED ? sign * x0 : x0, SIGNED ? sign * x1 : x1, h[u], m[u], l[u]);
+      }
       char* p = L + at(row, k >> 3) + (k & 7) * 2;
       put(p, h, W);
       put(p + PLANE, m, W);
@@ -730,6 +734,11 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
   const int lrow = lane % 32, h = lane / 32;
   // The stage in buffer P is multiplied while the next is split into the other buffer and the third from here loaded.
   // FRESH: the running sums take the last stages' part and a new one begins.
+  // The bf16 MFMAs round towards one side by a little (2^-27 of a part), which over thousands of k of terms of either
+  // sign would be most of the error. So every other part is made of a negated operand (the one of fewer rows), and the
+  // running sums change sign each time: [256, 65536] x [65536, 256] is 1.83e-7 from its f64 value so, 3.9e-7 without.
+  constexpr bool SIGNA = TA::PER <= TB::PER;
+  auto sign = [](int st) { return (st & 2) ? -1.0f : 1.0f; };
   auto body = [&](int st, auto ptag, auto ftag) {
     constexpr int P = decltype(ptag)::value;
     constexpr bool FRESH = decltype(ftag)::value != 0;
@@ -748,14 +757,14 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
     for (int j = 1; j < TN; ++j)
 #pragma unroll
       for (int o = 0; o < 3; ++o) bb[OB[o]][j] = TB::frag(Lb, OB[o], wn0 + j * 32 + lrow, h);
-    TA::store(qa[P ^ 1], mine + (P ^ 1) * BUF, tid);
-    TB::store(qb[P ^ 1], mine + (P ^ 1) * BUF + TA::SIZE, tid);
+    TA::template store<SIGNA>(qa[P ^ 1], mine + (P ^ 1) * BUF, tid, sign(st + 1));
+    TB::template store<!SIGNA>(qb[P ^ 1], mine + (P ^ 1) * BUF + TA::SIZE, tid, sign(st + 1));
     ahead(st + 3, P ^ 1);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if (FRESH) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) acc[i][j] += part[i][j];
+        for (int i = 0; i < TM; ++i) acc[i][j] = part[i][j] - acc[i][j];
       }
 #pragma unroll
       for (int t = 0; t < 6; ++t)
@@ -774,8 +783,8 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
       TB::mask(qb[0], keep, tid);
     }
     ahead(1, 1);
-    TA::store(qa[0], mine, tid);
-    TB::store(qb[0], mine + TA::SIZE, tid);
+    TA::template store<false>(qa[0], mine, tid, 1.0f);
+    TB::template store<false>(qb[0], mine + TA::SIZE, tid, 1.0f);
     ahead(2, 0);
   }
   meet();
@@ -789,7 +798,7 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] += part[i][j];
+    for (int j = 0; j < TN; ++j) acc[i][j] = (part[i][j] - acc[i][j]) * sign(cnt - 1);   // (by element: spills)
   if (KG > 1) {
     float* X = reinterpret_cast<float*>(lds);   // every group has passed its last read of the buffers
     if (kg > 0) {

@@ -373,7 +373,7 @@ int64_t x3_tiles(const XTiling& t, const GemmDesc& d) {
 
 // Longest k range that one group sums: the running sum of a range takes an addition per 32 k, the f32 tiles' (two
 // running sums over each split of plan_for) one per 64 or 128. Error variance against 64 bits, in units of 1e-14:
-// 0.5 + 1.2e-3 k here, 1.15 + 0.52e-3 k there; this keeps the first below the second.
+// at most 0.5 + 1.2e-3 k here, 1.15 + 0.52e-3 k there; this keeps the first below the second.
 int64_t x3_range(const GemmDesc& d) { return 512 + (int64_t)(0.4 * (double)plan_for(d).kps); }
 
 struct XPlan { int tiling, splits; int64_t kps; double us; };
