@@ -9,16 +9,15 @@
 //   conv2d_weight_grad dW[co][n=(cl,kh,kw)] = sum_{k=(b,p)} dy[b, co, p] * x[b, cl, ho*sH+kh-pH, wo*sW+kw-pW]
 // with p = (ho, wo), q = (hi, wi). Out-of-image taps read as zero.
 //
-// The gathers are separable: an operand element's offset is a term of its row (an output position, a weight row) plus a
-// term of its reduction index, and whether a tap falls outside the image is a bit of the position's row mask or column
-// mask, picked by the tap. Row terms are found once per block. The reduction index' terms (KTerm) are found once per
-// block and stage and read from LDS by all, so an element costs one add and, where taps can fall outside, three more
-// operations. Offsets are bytes modulo 2^32: every tensor has fewer than 2^29 elements, row terms are not
-// negative, so a valid sum is exact and an element that reads as zero gets bit 31 set, which the buffer unit returns 0 for.
-//
-// The input gradient of a strided convolution is one stride-1 problem per phase (hi mod sH, wi mod sW): the positions
-// of a phase meet the same taps, kh = kh0 + j * sH, and ho = hi' + dh - j, so no products with zeros are made. Its
-// reduction runs tap by tap, k = tap * CoutPG + col.
+// The gathers are separable: the element offset is (a term of the output position) + (a
+// term of the reduction index), e.g. for conv2d x offset = [b*Cin*HW + ho*sH*W + wo*sW]
+// + [cl*HW + (kh-pH)*W + (kw-pW)]. Each thread computes the terms of the output positions
+// it loads once per block and the terms of its k values once per stage, so a stage costs
+// one add and (with padding) two unsigned compares per element. Offsets are 32-bit
+// (every tensor has fewer than 2^29 elements; sums of a non-negative position term and a
+// possibly negative k term are taken modulo 2^32, which is exact for in-range results).
+// The input gradient with a stride above 1 uses a slower per-element map (divisibility
+// of hi + pH - kh by sH).
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -33,26 +32,28 @@ using gd::f32x4;
 #define CG_HD __host__ __device__ __forceinline__
 
 constexpr int kCT = 256;    // threads per block
-constexpr int kCBK = 16;    // k per LDS stage
+constexpr int kCBK = 32;    // k per LDS stage
+constexpr int kTab = 1024;  // conv2d / input gradient: k terms kept in an LDS table when K <= kTab
 
 enum { CV_FWD = 0, CV_DGRAD = 1, CV_WGRAD = 2 };
 // Loader variants, chosen per launch (template flags, so the k loop has no runtime tests):
-// F_AVEC: 4 consecutive k of A are consecutive in memory (one 16-byte load). F_PAD: some tap falls outside the image.
-// F_WIDE: a kernel of more than 32 rows or columns, whose taps do not fit the masks: coordinates are compared. F_TAP: a
-// thread's consecutive k share a tap (the input gradient over a multiple of 8 channels): one test for all.
-// F_BVEC: the weight gradient's 4 consecutive k of B are consecutive in memory (stride 1, no padding, Wo % 4 == 0).
-enum { F_AVEC = 1, F_PAD = 2, F_WIDE = 4, F_TAP = 8, F_BVEC = 16 };
+// F_AVEC: A rows are 16-byte aligned groups of 4 k (vector loads); F_TAB: the k terms come
+// from the block's LDS table; F_PAD: some tap falls outside the image (bounds checks);
+// F_TAP: conv2d or the stride-1 input gradient with a multiple of kCBK channels per group
+// runs its reduction tap-major, k = tap * channels + channel, so every stage holds one tap
+// and 32 channels: a thread finds its positions' offsets and in-image tests once per stage
+// and each element costs one add (the GEMM's k order changes, its value does not).
+enum { F_AVEC = 1, F_TAB = 2, F_PAD = 4, F_TAP = 8 };
 
 struct ConvGemmArgs {
   int B, Cin, H, W, Cout, CinPG, CoutPG, kH, kW, Ho, Wo, G, sH, sW, pH, pW;
   int M, N, K;                  // GEMM sizes per group
   int tiles_m, tiles_n, splits, k_per_split;
   int pad;                      // some tap can fall outside the image: bounds checks needed
-  int phases;                   // input gradient: min(sH, H) * min(sW, W)
+  int avec;                     // A rows are 16-byte aligned in groups of 4 k (vector loads)
   int ipb;                      // few-taps weight gradient: images per block
-  FastDiv dKHW, dKW, dWo, dHoWo;
-  FastDiv dCpg;                 // CoutPG
-  FastDiv dTn, dPh, dPhW;       // tiles_n; the input gradient's phases, and those of a row
+  FastDiv dKHW, dKW, dWo, dHoWo, dW, dHW, dSH, dSW;
+  FastDiv dCpg;                 // F_TAP: channels per group of the reduction (CinPG / CoutPG)
   const float* x;
   const float* w;
   const float* dy;
@@ -79,8 +80,9 @@ CG_HD bool inside(int a, int lim) { return (uint32_t)a < (uint32_t)lim; }
 
 // An operand tensor read through the buffer unit (raw buffer loads: 32-bit byte offsets
 // from a uniform base, and offsets at or past the tensor's size read as 0 without a
-// memory access). Elements that read as zero are loaded from an offset with bit 31 set, past
-// every tensor (fewer than 2^29 elements each), so the loads need no branches. The host build (used to exercise the loaders on the CPU) reads the
+// memory access). Masked elements are loaded from offset kMasked, so the loads need no
+// branches. Tensors have fewer than 2^29 elements, so kMasked lies past every tensor and
+// is 16-byte aligned. The host build (used to exercise the loaders on the CPU) reads the
 // array directly with the same rule.
 constexpr uint32_t kMasked = 0x80000000u;
 struct Src {
@@ -109,8 +111,7 @@ CG_HD float ldb(const Src& s, uint32_t off) {
   return off < s.bytes ? s.p[off >> 2] : 0.0f;
 #endif
 }
-CG_HD uint32_t boff(bool ok, uint32_t idx) { return ok ? idx << 2 : kMasked; }
-CG_HD f32x4 ldb4(const Src& s, uint32_t off) {   // off 4-byte aligned; all four elements inside or off >= kMasked
+CG_HD f32x4 ldb4(const Src& s, uint32_t off) {   // off 16-byte aligned
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(s.r, (int)off, 0, 0));
 #else
@@ -119,248 +120,341 @@ CG_HD f32x4 ldb4(const Src& s, uint32_t off) {   // off 4-byte aligned; all four
   return v;
 #endif
 }
+CG_HD uint32_t boff(bool ok, uint32_t idx) { return ok ? idx << 2 : kMasked; }
 
-// Bits [lo, hi) of the taps 0 .. n-1 at coordinates first + t (step > 0) or first - t (step < 0) that lie inside
-// 0 .. lim-1 are clear, the others set (n <= 32).
-CG_HD uint32_t outside_bits(int first, int step, int n, int lim) {
-  const int lo = std::max(0, step > 0 ? -first : first - lim + 1);
-  const int hi = std::min(n, step > 0 ? lim - first : first + 1);
-  return hi <= lo ? ~0u : ~((~0u >> (32 - (hi - lo))) << lo);
+// k term of conv2d / the stride-1 input gradient for reduction index k: the offset term
+// and the two spatial shifts packed as 16-bit halves (low: row shift, high: column shift).
+CG_HD void k_term(const ConvGemmArgs& c, int mode, int k, uint32_t& off, uint32_t& shifts) {
+  const int khw = c.kH * c.kW;
+  const int kc = fdiv(k, c.dKHW), r = k - kc * khw;
+  const int kh = fdiv(r, c.dKW), kw = r - kh * c.kW;
+  int a, b;
+  if (mode == CV_FWD) {
+    a = kh - c.pH;
+    b = kw - c.pW;
+    off = (uint32_t)(kc * c.H * c.W) + (uint32_t)(a * c.W + b);
+  } else {
+    a = kh;
+    b = kw;
+    off = (uint32_t)(kc * c.Ho * c.Wo) - (uint32_t)(kh * c.Wo + kw);
+  }
+  shifts = ((uint32_t)a & 0xFFFFu) | ((uint32_t)b << 16);
+}
+CG_HD int shift_lo(uint32_t s) { return (int)(int16_t)(s & 0xFFFFu); }
+CG_HD int shift_hi(uint32_t s) { return (int)(int16_t)(s >> 16); }
+
+// Block position in the launch grid: output tile (tm, tn), group z and k split.
+struct BlockPos {
+  int m0, n0, z, split, kbeg, kend;
+};
+
+template <int BM, int BN>
+CG_HD BlockPos block_pos(const ConvGemmArgs& c, uint32_t blk, uint32_t nblk, int mode) {
+  // Tiles are numbered so each XCD (the chip's 8 L2 domains take blocks round robin)
+  // receives a contiguous run, n fastest.
+  uint32_t bid = blk;
+  if (nblk % gd::kXcds == 0) bid = (bid % gd::kXcds) * (nblk / gd::kXcds) + bid / gd::kXcds;
+  BlockPos p;
+  const int tn = bid % c.tiles_n;
+  const uint32_t rest = bid / c.tiles_n;
+  const int tm = rest % c.tiles_m;
+  const int zs = rest / c.tiles_m;
+  p.m0 = tm * BM;
+  p.n0 = tn * BN;
+  p.z = mode == CV_WGRAD ? zs / c.splits : zs;
+  p.split = mode == CV_WGRAD ? zs % c.splits : 0;
+  p.kbeg = p.split * c.k_per_split;
+  p.kend = std::min(c.K, p.kbeg + c.k_per_split);
+  return p;
 }
 
-// The term of reduction index k: byte offsets into A and B, and the two numbers that the in-image test takes from the
-// reduction side. conv2d and the input gradient: shifts 31 - tap row / column, which bring the row term's mask bits to
-// bit 31 (F_WIDE: the tap's row / column shift). Weight gradient: the position's masks (F_WIDE: its coordinates).
-struct KTerm { uint32_t a, b, t0, t1; };
-// The term of a row of B (conv2d, input gradient: an output position; weight gradient: a tap of a channel).
-struct BTerm { uint32_t off, t0, t1; };
+// Register-staged coordinates of element group `e` of thread `tid` (as k_gemm's Tile):
+// k-contiguous operands take 4 consecutive k of one row, row-contiguous ones 4
+// consecutive rows at one k.
+template <int ROWS, bool KFAST, int E>
+CG_HD void stage_coords(int tid, int& rr, int& kk) {
+  const int idx = tid + E * kCT;
+  if (KFAST) { rr = idx / (kCBK / 4); kk = (idx % (kCBK / 4)) * 4; }
+  else { rr = (idx % (ROWS / 4)) * 4; kk = idx / (ROWS / 4); }
+}
 
-// One output tile's place and the maps of one launch's operands.
-template <int MODE, int F>
-struct ConvMap {
-  int m0, n0, z, split, kbeg, kend;   // tile origin, group, k range
-  int N;                              // columns (input gradient: of the phase)
-  // input gradient's phase: first position, position grid, first tap, taps, output row of (hi' = 0, tap 0)
-  int rh, rw, Hr, Wr, kh0, kw0, nh, nw, dh, dw;
-  int rnw;                            // 65536 / nw, rounded up
-  Src sa, sb;
+// Per-thread loader of one block's operand stages. MODE selects the convolution kind;
+// FAST = the separable maps (conv2d always, the input gradient at stride 1, the weight
+// gradient always).
+template <int MODE, bool FAST, int BM, int BN, int F>
+struct ConvLoader {
+  static constexpr bool BKF = MODE == CV_WGRAD;          // B staged k-contiguous
+  static constexpr int QA = BM * kCBK / (4 * kCT);
+  static constexpr int QB = BN * kCBK / (4 * kCT);
+  BlockPos bp;
+  int tid;
+  Src sx, sw, sdy;  // x, w, dy
+  // row-contiguous B (conv2d, input gradient): the thread's 4 output positions
+  uint32_t nb[4];   // position term of the offset
+  int ph[4], pw[4]; // spatial coordinates the k term's (dh, dw) is added to
+  int nvalid;       // bit u: position u exists
+  // k-contiguous B (weight gradient): the thread's output columns n, one per group
+  uint32_t wnoff[QB > 0 ? QB : 1];
+  int wdh[QB > 0 ? QB : 1], wdw[QB > 0 ? QB : 1];
+  int wnvalid;      // bit e: column of group e exists
 
-  template <int BM, int BN>
-  CG_HD void init(const ConvGemmArgs& c, uint32_t blk, uint32_t nblk) {
-    // Tiles are numbered so each XCD (the chip's 8 L2 domains take blocks round robin) receives a contiguous run, n
-    // fastest (input gradient: phase fastest, so that a run holds as many blocks of each).
-    uint32_t bid = blk;
-    if (nblk % gd::kXcds == 0) bid = (bid % gd::kXcds) * (nblk / gd::kXcds) + bid / gd::kXcds;
-    const int rest = fdiv((int)bid, c.dTn);
-    int tn = (int)bid - rest * c.tiles_n;
-    const int tm = rest % c.tiles_m, zs = rest / c.tiles_m;
-    m0 = tm * BM;
-    z = MODE == CV_WGRAD ? zs / c.splits : zs;
-    split = MODE == CV_WGRAD ? zs % c.splits : 0;
-    kbeg = split * c.k_per_split;
-    kend = std::min(c.K, kbeg + c.k_per_split);
-    N = c.N;
-    if (MODE == CV_DGRAD) {
-      const int t = fdiv(tn, c.dPh), ph = tn - t * c.phases;
-      tn = t;
-      rh = fdiv(ph, c.dPhW);
-      rw = ph - rh * (int)c.dPhW.d;
-      Hr = (c.H - rh + c.sH - 1) / c.sH;
-      Wr = (c.W - rw + c.sW - 1) / c.sW;
-      kh0 = (rh + c.pH) % c.sH;
-      kw0 = (rw + c.pW) % c.sW;
-      nh = (c.kH - kh0 + c.sH - 1) / c.sH;   // (kh0 < sH: not negative)
-      nw = (c.kW - kw0 + c.sW - 1) / c.sW;
-      rnw = 65536 / std::max(nw, 1) + 1;
-      dh = (rh + c.pH - kh0) / c.sH;
-      dw = (rw + c.pW - kw0) / c.sW;
-      N = c.B * Hr * Wr;
-      kend = nh * nw * c.CoutPG;
-    }
-    n0 = tn * BN;
-    const int64_t xs = (int64_t)c.B * c.Cin * c.H * c.W, ws = (int64_t)c.Cout * c.CinPG * c.kH * c.kW,
-                  ys = (int64_t)c.B * c.Cout * c.Ho * c.Wo;
-    if (MODE == CV_FWD) { sa = make_src(c.w, ws); sb = make_src(c.x, xs); }
-    else if (MODE == CV_DGRAD) { sa = make_src(c.w, ws); sb = make_src(c.dy, ys); }
-    else { sa = make_src(c.dy, ys); sb = make_src(c.x, xs); }
-  }
-
-  // Position of column n: image, row, column of the output (input gradient: in the phase's grid).
-  CG_HD void position(const ConvGemmArgs& c, int n, int& b, int& i, int& j) const {
-    if (MODE == CV_DGRAD) {
-      const int hw = Hr * Wr;
-      b = n / hw;
-      const int q = n - b * hw;
-      i = q / Wr;
-      j = q - i * Wr;
+  CG_HD void init(const ConvGemmArgs& c, const BlockPos& p, int t) {
+    bp = p;
+    tid = t;
+    sx = make_src(c.x, (int64_t)c.B * c.Cin * c.H * c.W);
+    sw = make_src(c.w, (int64_t)c.Cout * c.CinPG * c.kH * c.kW);
+    sdy = make_src(c.dy, (int64_t)c.B * c.Cout * c.Ho * c.Wo);
+    nvalid = 0;
+    wnvalid = 0;
+    if (!BKF) {
+      int rr, kk;
+      stage_coords<BN, false, 0>(tid, rr, kk);   // every group of a thread has the same rows
+      const int n0 = p.n0 + rr;
+      const int g = p.z;
+      if (MODE == CV_FWD) {
+        const int hw = c.Ho * c.Wo;
+        int b = n0 < c.N ? fdiv(n0, c.dHoWo) : 0;
+        int q = n0 - b * hw;
+        int ho = fdiv(q, c.dWo), wo = q - ho * c.Wo;
+        for (int u = 0; u < 4; ++u) {
+          if (n0 + u < c.N) {
+            nvalid |= 1 << u;
+            nb[u] = (uint32_t)(((b * c.Cin + g * c.CinPG) * c.H + ho * c.sH) * c.W + wo * c.sW);
+            ph[u] = ho * c.sH;
+            pw[u] = wo * c.sW;
+          } else {
+            nb[u] = 0; ph[u] = 0; pw[u] = 0;
+          }
+          if (++wo == c.Wo) { wo = 0; if (++ho == c.Ho) { ho = 0; ++b; } }
+        }
+      } else {   // CV_DGRAD: positions (b, hi, wi) of dX
+        const int hw = c.H * c.W;
+        int b = n0 < c.N ? fdiv(n0, c.dHW) : 0;
+        int q = n0 - b * hw;
+        int hi = fdiv(q, c.dW), wi = q - hi * c.W;
+        for (int u = 0; u < 4; ++u) {
+          if (n0 + u < c.N) {
+            nvalid |= 1 << u;
+            // stride 1: ho = hi + pH - kh, wo = wi + pW - kw
+            nb[u] = (uint32_t)(((b * c.Cout + g * c.CoutPG) * c.Ho + hi + c.pH) * c.Wo + wi + c.pW);
+            ph[u] = FAST ? hi + c.pH : hi;
+            pw[u] = FAST ? wi + c.pW : wi;
+          } else {
+            nb[u] = 0; ph[u] = 0; pw[u] = 0;
+          }
+          if (++wi == c.W) { wi = 0; if (++hi == c.H) { hi = 0; ++b; } }
+        }
+      }
     } else {
-      b = fdiv(n, c.dHoWo);
-      const int q = n - b * c.Ho * c.Wo;
-      i = fdiv(q, c.dWo);
-      j = q - i * c.Wo;
+      const int khw = c.kH * c.kW;
+      for (int e = 0; e < QB; ++e) {
+        int rr, kk;
+        stage_coords_rt(e, rr, kk);
+        const int n = p.n0 + rr;
+        if (n < c.N) {
+          wnvalid |= 1 << e;
+          const int cl = fdiv(n, c.dKHW), r = n - cl * khw;
+          const int kh = fdiv(r, c.dKW), kw = r - kh * c.kW;
+          wdh[e] = kh - c.pH;
+          wdw[e] = kw - c.pW;
+          wnoff[e] = (uint32_t)(((p.z * c.CinPG + cl) * c.H) * c.W) + (uint32_t)(wdh[e] * c.W + wdw[e]);
+        } else {
+          wdh[e] = 0; wdw[e] = 0; wnoff[e] = 0;
+        }
+      }
     }
   }
 
-  // Byte offset term of row m of A (past the last row: the last).
-  CG_HD uint32_t a_row(const ConvGemmArgs& c, int m) const {
-    const int mm = std::min(m, c.M - 1);
-    if (MODE == CV_FWD) return (uint32_t)((z * c.CoutPG + mm) * c.K) << 2;
-    if (MODE == CV_DGRAD) return (uint32_t)((z * c.CoutPG * c.CinPG + mm) * c.kH * c.kW) << 2;
-    return (uint32_t)((z * c.CoutPG + mm) * c.Ho * c.Wo) << 2;
+  // Runtime-index version of stage_coords for the KFAST B operand.
+  CG_HD void stage_coords_rt(int e, int& rr, int& kk) const {
+    const int idx = tid + e * kCT;
+    rr = idx / (kCBK / 4);
+    kk = (idx % (kCBK / 4)) * 4;
   }
 
-  // The term of row n of B (past the last: the last; its products are not stored).
-  CG_HD BTerm b_row(const ConvGemmArgs& c, int n) const {
-    BTerm t;
-    const int nn = std::min(n, N - 1);
-    if (MODE == CV_WGRAD) {
-      const int cl = fdiv(nn, c.dKHW), r = nn - cl * c.kH * c.kW;
-      const int kh = fdiv(r, c.dKW), kw = r - kh * c.kW;
-      t.off = (uint32_t)(((z * c.CinPG + cl) * c.H + kh) * c.W + kw) << 2;
-      t.t0 = (F & F_WIDE) ? kh : 31 - kh;
-      t.t1 = (F & F_WIDE) ? kw : 31 - kw;
-      return t;
-    }
-    int b, i, j;
-    position(c, nn, b, i, j);
-    if (MODE == CV_FWD) {
-      t.off = (uint32_t)(((b * c.Cin + z * c.CinPG) * c.H + i * c.sH) * c.W + j * c.sW) << 2;
-      t.t0 = (F & F_WIDE) ? i * c.sH - c.pH : outside_bits(i * c.sH - c.pH, 1, c.kH, c.H);
-      t.t1 = (F & F_WIDE) ? j * c.sW - c.pW : outside_bits(j * c.sW - c.pW, 1, c.kW, c.W);
-    } else {
-      t.off = (uint32_t)(((b * c.Cout + z * c.CoutPG) * c.Ho + i + dh) * c.Wo + j + dw) << 2;
-      t.t0 = (F & F_WIDE) ? i + dh : outside_bits(i + dh, -1, nh, c.Ho);
-      t.t1 = (F & F_WIDE) ? j + dw : outside_bits(j + dw, -1, nw, c.Wo);
-    }
-    return t;
-  }
-
-  CG_HD KTerm k_term(const ConvGemmArgs& c, int k) const {
-    KTerm t;
-    if (k >= kend) {   // both operands read as zero
-      t.a = t.b = kMasked;
-      t.t0 = t.t1 = 0;
-      return t;
+  // A operand (always k-contiguous): 4 consecutive k of row m.
+  CG_HD f32x4 load_a(const ConvGemmArgs& c, int m, int k0) const {
+    f32x4 v;
+    const int kend = bp.kend;
+    const bool mok = m < c.M;
+    const int mm = mok ? m : 0;
+    if ((F & F_TAP) && MODE != CV_WGRAD) {
+      // k = tap * cpg + ch; the 4 k share the tap (cpg % 4 == 0, k0 % 4 == 0) and lie below
+      // kend (K = taps * cpg, a multiple of kCBK). Consecutive channels are a fixed stride
+      // apart in the weight.
+      const int khw = c.kH * c.kW;
+      const int cpg = MODE == CV_FWD ? c.CinPG : c.CoutPG;
+      const int tap = fdiv(k0, c.dCpg), ch = k0 - tap * cpg;
+      const uint32_t o = MODE == CV_FWD ? (uint32_t)(((bp.z * c.CoutPG + mm) * c.CinPG + ch) * khw + tap)
+                                        : (uint32_t)(((bp.z * c.CoutPG + ch) * c.CinPG + mm) * khw + tap);
+      const uint32_t step = MODE == CV_FWD ? (uint32_t)khw : (uint32_t)(c.CinPG * khw);
+      for (int u = 0; u < 4; ++u) v[u] = ldb(sw, mok ? (o + u * step) << 2 : kMasked);
+      (void)kend;
+      return v;
     }
     if (MODE == CV_FWD) {
-      const int cl = fdiv(k, c.dKHW), r = k - cl * c.kH * c.kW;
-      const int kh = fdiv(r, c.dKW), kw = r - kh * c.kW;
-      t.a = (uint32_t)k << 2;
-      t.b = (uint32_t)((cl * c.H + kh - c.pH) * c.W + kw - c.pW) << 2;
-      t.t0 = (F & F_WIDE) ? kh : 31 - kh;
-      t.t1 = (F & F_WIDE) ? kw : 31 - kw;
+      const uint32_t row = (uint32_t)((bp.z * c.CoutPG + mm) * c.K);
+      // avec: K % 4 == 0 and k0 % 4 == 0, so k0 < kend covers all 4
+      if (F & F_AVEC) return ldb4(sw, boff(mok && k0 < kend, row + (uint32_t)k0));
+      for (int u = 0; u < 4; ++u) v[u] = ldb(sw, boff(mok && k0 + u < kend, row + (uint32_t)(k0 + u)));
     } else if (MODE == CV_DGRAD) {
-      const int tap = fdiv(k, c.dCpg), col = k - tap * c.CoutPG;
-      // (fewer than 1024 taps, nw <= 32: rnw * nw - 65536 < 32, so the quotient is exact)
-      const int jh = (F & F_WIDE) ? tap / nw : (int)((uint32_t)(tap * rnw) >> 16), jw = tap - jh * nw;
-      t.a = (uint32_t)((col * c.CinPG * c.kH + kh0 + jh * c.sH) * c.kW + kw0 + jw * c.sW) << 2;
-      t.b = (uint32_t)((col * c.Ho - jh) * c.Wo - jw) << 2;
-      t.t0 = (F & F_WIDE) ? -jh : 31 - jh;
-      t.t1 = (F & F_WIDE) ? -jw : 31 - jw;
+      const int khw = c.kH * c.kW;
+      int col = fdiv(k0, c.dKHW), r = k0 - col * khw;
+      for (int u = 0; u < 4; ++u) {
+        const bool ok = mok && k0 + u < kend;
+        v[u] = ldb(sw, boff(ok, (uint32_t)(((bp.z * c.CoutPG + (ok ? col : 0)) * c.CinPG + mm) * khw + r)));
+        if (++r == khw) { r = 0; ++col; }
+      }
+    } else {   // CV_WGRAD: dy[b, co, p] for k = (b, p)
+      const int hw = c.Ho * c.Wo;
+      const bool kok = k0 < kend;
+      int b = kok ? fdiv(k0, c.dHoWo) : 0, p = kok ? k0 - b * hw : 0;
+      // avec: hw % 4 == 0 and k0 % 4 == 0, so the 4 k lie in one image, 16-byte aligned
+      if (F & F_AVEC) return ldb4(sdy, boff(mok && kok, (uint32_t)((b * c.Cout + bp.z * c.CoutPG + mm) * hw + p)));
+      for (int u = 0; u < 4; ++u) {
+        const bool ok = mok && k0 + u < kend;
+        v[u] = ldb(sdy, boff(ok, (uint32_t)(((ok ? b : 0) * c.Cout + bp.z * c.CoutPG + mm) * hw + (ok ? p : 0))));
+        if (++p == hw) { p = 0; ++b; }
+      }
+    }
+    return v;
+  }
+
+  // Row-contiguous B (conv2d, input gradient): the thread's 4 positions at one k. `tab`
+  // holds (offset, shifts) of every k when K <= kTab (else null: computed here).
+  CG_HD f32x4 load_b_rows(const ConvGemmArgs& c, int k, const uint32_t* tab) const {
+    f32x4 v;
+    const bool kok = k < bp.kend;
+    const int kq = kok ? k : 0;
+    if (MODE == CV_FWD || FAST) {
+      uint32_t koff, sh;
+      if (F & F_TAB) { koff = tab[2 * kq]; sh = tab[2 * kq + 1]; }
+      else k_term(c, MODE, kq, koff, sh);
+      const int a = shift_lo(sh), b = shift_hi(sh);
+      const Src& src = MODE == CV_FWD ? sx : sdy;
+      for (int u = 0; u < 4; ++u) {
+        bool ok = kok && ((nvalid >> u) & 1);
+        if (MODE == CV_FWD) {
+          if (F & F_PAD) ok = ok && inside(ph[u] + a, c.H) && inside(pw[u] + b, c.W);
+        } else {
+          ok = ok && inside(ph[u] - a, c.Ho) && inside(pw[u] - b, c.Wo);
+        }
+        v[u] = ldb(src, boff(ok, nb[u] + koff));
+      }
+    } else {             // input gradient, any stride: ph / pw hold (hi, wi)
+      const int khw = c.kH * c.kW;
+      const int kc = fdiv(kq, c.dKHW), r = kq - kc * khw;
+      const int kh = fdiv(r, c.dKW), kw = r - kh * c.kW;
+      for (int u = 0; u < 4; ++u) {
+        const int nh = ph[u] + c.pH - kh, nw = pw[u] + c.pW - kw;
+        bool ok = kok && ((nvalid >> u) & 1) && nh >= 0 && nw >= 0;
+        const int ho = fdiv(ok ? nh : 0, c.dSH), wo = fdiv(ok ? nw : 0, c.dSW);
+        ok = ok && ho * c.sH == nh && wo * c.sW == nw && ho < c.Ho && wo < c.Wo;
+        // nb[u] - (hi + pH) * Wo - (wi + pW) is the (b, g) plane base
+        const uint32_t plane = nb[u] - (uint32_t)((ph[u] + c.pH) * c.Wo + pw[u] + c.pW);
+        v[u] = ldb(sdy, boff(ok, plane + (uint32_t)(kc * c.Ho * c.Wo + ho * c.Wo + wo)));
+      }
+    }
+    return v;
+  }
+
+  // k-contiguous B (weight gradient): group e's column at 4 consecutive k = (b, ho, wo).
+  // kb/khs/kws: the per-stage k terms (position term, spatial coordinates) of the 4 k.
+  CG_HD f32x4 load_b_cols(const ConvGemmArgs& c, int e, const uint32_t* kb, const int* khs, const int* kws,
+                          int kmask) const {
+    f32x4 v;
+    const bool nok = (wnvalid >> e) & 1;
+    for (int u = 0; u < 4; ++u) {
+      bool ok = nok && ((kmask >> u) & 1);
+      if (F & F_PAD) ok = ok && inside(khs[u] + wdh[e], c.H) && inside(kws[u] + wdw[e], c.W);
+      v[u] = ldb(sx, boff(ok, kb[u] + wnoff[e]));
+    }
+    return v;
+  }
+
+  // One stage: fill qa[QA] / qb[QB] with the elements this thread stages for k0.
+  CG_HD void load(const ConvGemmArgs& c, int k0, f32x4* qa, f32x4* qb, const uint32_t* tab) const {
+    for (int e = 0; e < QA; ++e) {
+      const int idx = tid + e * kCT;
+      const int rr = idx / (kCBK / 4), kk = (idx % (kCBK / 4)) * 4;
+      qa[e] = load_a(c, bp.m0 + rr, k0 + kk);
+    }
+    if (!BKF && (F & F_TAP)) {
+      // The stage's 32 k are one tap (cpg % kCBK == 0, k0 % kCBK == 0, K = taps * cpg, so
+      // every k < kend): in-image tests and offset bases per position once, then per k the
+      // channel's plane offset. Masked positions keep the out-of-range base kMasked, which
+      // the added plane offset (below 2^31 bytes) leaves out of range.
+      const int cpg = MODE == CV_FWD ? c.CinPG : c.CoutPG;
+      const int tap = fdiv(k0, c.dCpg);
+      const int kh = fdiv(tap, c.dKW), kw = tap - kh * c.kW;
+      const int a = MODE == CV_FWD ? kh - c.pH : kh, b = MODE == CV_FWD ? kw - c.pW : kw;
+      const uint32_t toff = MODE == CV_FWD ? (uint32_t)(a * c.W + b) : (uint32_t)0 - (uint32_t)(kh * c.Wo + kw);
+      const uint32_t plane = MODE == CV_FWD ? (uint32_t)(c.H * c.W) : (uint32_t)(c.Ho * c.Wo);
+      const Src& src = MODE == CV_FWD ? sx : sdy;
+      uint32_t base[4];
+      for (int u = 0; u < 4; ++u) {
+        bool ok = (nvalid >> u) & 1;
+        if (MODE == CV_FWD) {
+          if (F & F_PAD) ok = ok && inside(ph[u] + a, c.H) && inside(pw[u] + b, c.W);
+        } else {
+          ok = ok && inside(ph[u] - a, c.Ho) && inside(pw[u] - b, c.Wo);
+        }
+        base[u] = ok ? (nb[u] + toff) << 2 : kMasked;
+      }
+      const int ch0 = k0 - tap * cpg;
+      for (int e = 0; e < QB; ++e) {
+        const int kk = (tid + e * kCT) / (BN / 4);
+        const uint32_t delta = ((uint32_t)(ch0 + kk) * plane) << 2;
+        for (int u = 0; u < 4; ++u) qb[e][u] = ldb(src, base[u] + delta);
+      }
+    } else if (!BKF) {
+      for (int e = 0; e < QB; ++e) {
+        const int idx = tid + e * kCT;
+        const int kk = idx / (BN / 4);
+        qb[e] = load_b_rows(c, k0 + kk, tab);
+      }
     } else {
-      const int b = fdiv(k, c.dHoWo), p = k - b * c.Ho * c.Wo;
-      const int ho = fdiv(p, c.dWo), wo = p - ho * c.Wo;
-      const int h = ho * c.sH - c.pH, w = wo * c.sW - c.pW;
-      t.a = (uint32_t)(b * c.Cout * c.Ho * c.Wo + p) << 2;
-      t.b = (uint32_t)((b * c.Cin * c.H + h) * c.W + w) << 2;
-      t.t0 = (F & F_WIDE) ? h : outside_bits(h, 1, c.kH, c.H);
-      t.t1 = (F & F_WIDE) ? w : outside_bits(w, 1, c.kW, c.W);
+      // The thread's 4 k are the same for every group (kk depends on tid only).
+      const int kk = (tid % (kCBK / 4)) * 4;
+      uint32_t kb[4];
+      int khs[4], kws[4], kmask = 0;
+      const int hw = c.Ho * c.Wo;
+      const int ks = k0 + kk;
+      int b = 0, p = 0;
+      if (ks < bp.kend) { b = fdiv(ks, c.dHoWo); p = ks - b * hw; }
+      int ho = fdiv(p, c.dWo), wo = p - ho * c.Wo;
+      for (int u = 0; u < 4; ++u) {
+        if (ks + u < bp.kend) kmask |= 1 << u;
+        kb[u] = (uint32_t)((b * c.Cin * c.H + ho * c.sH) * c.W + wo * c.sW);
+        khs[u] = ho * c.sH;
+        kws[u] = wo * c.sW;
+        if (++wo == c.Wo) { wo = 0; if (++ho == c.Ho) { ho = 0; ++b; } }
+      }
+      for (int e = 0; e < QB; ++e) qb[e] = load_b_cols(c, e, kb, khs, kws, kmask);
     }
-    return t;
   }
 
-  // Bit 31: the element of B at (row, k) lies outside the image.
-  CG_HD uint32_t outside(const ConvGemmArgs& c, uint32_t r0, uint32_t r1, uint32_t k0, uint32_t k1) const {
-    if (MODE != CV_DGRAD && !(F & F_PAD)) return 0;
-    if (F & F_WIDE) {
-      const int lh = MODE == CV_DGRAD ? c.Ho : c.H, lw = MODE == CV_DGRAD ? c.Wo : c.W;
-      return inside((int)(r0 + k0), lh) && inside((int)(r1 + k1), lw) ? 0u : kMasked;
+  // Output offset of GEMM element (0, gn) and the stride between rows gm (for split-K
+  // weight gradients, the offset inside the split's partial tile array).
+  CG_HD int64_t out_col(const ConvGemmArgs& c, int gn) const {
+    if (MODE == CV_FWD) {
+      const int hw = c.Ho * c.Wo;
+      const int b = fdiv(gn, c.dHoWo), q = gn - b * hw;
+      return ((int64_t)b * c.Cout + bp.z * c.CoutPG) * hw + q;
     }
-    if (MODE == CV_WGRAD) return ((k0 << (r0 & 31)) | (k1 << (r1 & 31))) & kMasked;
-    return ((r0 << (k0 & 31)) | (r1 << (k1 & 31))) & kMasked;
-  }
-
-  // Output offset of GEMM element (0, n) and the stride between rows m (for split weight gradients, the offset inside
-  // the split's partial tile array).
-  CG_HD int64_t out_col(const ConvGemmArgs& c, int n) const {
-    if (MODE == CV_WGRAD) return ((int64_t)(c.splits > 1 ? split * c.G : 0) + z) * c.M * c.N + n;
-    int b, i, j;
-    position(c, n, b, i, j);
-    if (MODE == CV_FWD) return (((int64_t)b * c.Cout + z * c.CoutPG) * c.Ho + i) * c.Wo + j;
-    return (((int64_t)b * c.Cin + z * c.CinPG) * c.H + i * c.sH + rh) * c.W + j * c.sW + rw;
+    if (MODE == CV_DGRAD) {
+      const int hw = c.H * c.W;
+      const int b = fdiv(gn, c.dHW), q = gn - b * hw;
+      return ((int64_t)b * c.Cin + bp.z * c.CinPG) * hw + q;
+    }
+    if (c.splits > 1) return ((int64_t)bp.split * c.G + bp.z) * c.M * c.N + gn;
+    return (int64_t)bp.z * c.M * c.N + gn;
   }
   CG_HD int64_t out_rs(const ConvGemmArgs& c) const {
     return MODE == CV_FWD ? (int64_t)c.Ho * c.Wo : MODE == CV_DGRAD ? (int64_t)c.H * c.W : (int64_t)c.N;
   }
 };
 
-// The 16 terms of a stage in LDS.
-struct KTab { uint32_t a[kCBK], b[kCBK], t0[kCBK], t1[kCBK]; };
-
-// What one thread loads of a stage. A: 4 k of a row (a tile of 32 rows: the first two wavefronts); in the input gradient
-// lanes take consecutive rows, kH * kW elements apart, since its consecutive k lie further apart. B, conv2d and
-// input gradient: PB consecutive k of row tid % BN, so a wavefront's loads take consecutive output positions. Weight
-// gradient: 4 k of rows tid / 4 + 64 e, whose consecutive k are consecutive positions.
-template <int MODE, int BM, int BN, int F>
-struct ConvLoader {
-  static constexpr bool ROWS = MODE != CV_WGRAD;
-  static constexpr int PB = BN * kCBK / kCT;          // elements of B per thread: 8 or 4
-  static constexpr int NR = ROWS ? 1 : PB / 4;        // its rows
-  uint32_t arow;
-  BTerm brow[NR];
-  int ka, kb;                                         // first k in the stage
-
-  CG_HD static int a_row(int tid) { return MODE == CV_DGRAD ? tid % BM : tid >> 2; }
-  CG_HD static int b_row(int tid, int e) { return ROWS ? tid % BN : (tid >> 2) + 64 * e; }
-
-  CG_HD void init(const ConvMap<MODE, F>& map, const ConvGemmArgs& c, int tid) {
-    arow = map.a_row(c, map.m0 + a_row(tid));
-    for (int e = 0; e < NR; ++e) brow[e] = map.b_row(c, map.n0 + b_row(tid, e));
-    ka = MODE == CV_DGRAD ? tid / BM * 4 & 12 : (tid & 3) * 4;
-    kb = ROWS ? tid / BN * PB : (tid & 3) * 4;
-  }
-  CG_HD void load(const ConvMap<MODE, F>& map, const ConvGemmArgs& c, const KTab& t, bool has_a, float* qa,
-                  float* qb) const {
-    if (has_a) {
-      if (F & F_AVEC) {
-        const f32x4 v = ldb4(map.sa, arow + t.a[ka]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) qa[u] = v[u];
-      } else {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) qa[u] = ldb(map.sa, arow + t.a[ka + u]);
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < NR; ++e) {
-      const BTerm& r = brow[e];
-      if (F & F_BVEC) {
-        const f32x4 v = ldb4(map.sb, r.off + t.b[kb]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) qb[e * 4 + u] = v[u];
-        continue;
-      }
-      if (F & F_TAP) {
-        // lanes outside the image take no part: as out-of-range loads they cost more (48 us in place of 44)
-#pragma unroll
-        for (int u = 0; u < PB; ++u) qb[u] = 0.0f;
-        if (map.outside(c, r.t0, r.t1, t.t0[kb], t.t1[kb]) == 0) {
-#pragma unroll
-          for (int u = 0; u < PB; ++u) qb[u] = ldb(map.sb, r.off + t.b[kb + u]);
-        }
-        continue;
-      }
-#pragma unroll
-      for (int u = 0; u < PB / NR; ++u) {
-        const int k = kb + u;
-        const uint32_t out = map.outside(c, r.t0, r.t1, t.t0[k], t.t1[k]);
-        qb[e * (PB / NR) + u] = ldb(map.sb, (r.off + t.b[k]) | out);
-      }
-    }
-  }
-};
-
-// (the tiles: see k_conv_gemm)
 struct ConvPlan { int mode, bm, bn, splits, k_per_split, tiles_m, tiles_n; int64_t blocks; };
 
 inline ConvPlan conv_plan(int mode, const ConvDesc& d) {
@@ -368,29 +462,28 @@ inline ConvPlan conv_plan(int mode, const ConvDesc& d) {
   p.mode = mode;
   const int64_t CoutPG = d.Cout / d.G, khw = d.kH * d.kW;
   const int64_t M = mode == CV_DGRAD ? d.CinPG : CoutPG;
-  // (input gradient: the columns of phase 0, the largest)
-  const int64_t N = mode == CV_FWD     ? d.B * d.Ho * d.Wo
-                    : mode == CV_DGRAD ? d.B * ((d.H + d.sH - 1) / d.sH) * ((d.W + d.sW - 1) / d.sW)
-                                       : d.CinPG * khw;
+  const int64_t N = mode == CV_FWD ? d.B * d.Ho * d.Wo : mode == CV_DGRAD ? d.B * d.H * d.W : d.CinPG * khw;
   const int64_t K = mode == CV_FWD ? d.CinPG * khw : mode == CV_DGRAD ? CoutPG * khw : d.B * d.Ho * d.Wo;
-  const int64_t Z = d.G, phases = mode == CV_DGRAD ? std::min(d.sH, d.H) * std::min(d.sW, d.W) : 1;
+  const int64_t Z = d.G;
+  // Tiles measured at the CNN config's shapes: 64 x 64 where M > 32 (more blocks in
+  // flight than 64 x 128 at the same per-element cost), 32 x 128 for 32-row outputs.
   p.bm = M <= 32 ? 32 : 64;
   p.bn = p.bm == 32 ? 128 : 64;
   p.tiles_m = (int)((M + p.bm - 1) / p.bm);
-  p.tiles_n = (int)((N + p.bn - 1) / p.bn * phases);
+  p.tiles_n = (int)((N + p.bn - 1) / p.bn);
   p.splits = 1;
   p.k_per_split = (int)K;
   if (mode == CV_WGRAD) {
-    // Enough blocks to fill the chip twice over, each split at least 256 k, and the
+    // Enough blocks to fill the chip twice over, each split at least 8 k stages, and the
     // partials within kConvWorkBytes.
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * Z;
     int64_t s = (512 + tiles - 1) / tiles;
-    s = std::min<int64_t>(s, std::max<int64_t>(1, K / 256));
+    s = std::min<int64_t>(s, std::max<int64_t>(1, K / (8 * kCBK)));
     const int64_t per = Z * M * N * 4;
     s = std::min<int64_t>(s, std::max<int64_t>(1, kConvWorkBytes / per));
     if (s > 1) {
       int64_t kps = (K + s - 1) / s;
-      kps = (kps + 31) / 32 * 32;
+      kps = (kps + kCBK - 1) / kCBK * kCBK;
       s = (K + kps - 1) / kps;
       p.k_per_split = (int)kps;
     }
@@ -411,28 +504,34 @@ inline ConvGemmArgs make_args(const ConvDesc& d, const ConvPlan& p) {
   else if (p.mode == CV_DGRAD) { a.M = a.CinPG; a.N = a.B * a.H * a.W; a.K = a.CoutPG * khw; }
   else { a.M = a.CoutPG; a.N = a.CinPG * khw; a.K = a.B * a.Ho * a.Wo; }
   a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.splits = p.splits; a.k_per_split = p.k_per_split;
-  a.phases = p.mode == CV_DGRAD ? std::min(a.sH, a.H) * std::min(a.sW, a.W) : 1;
   // A tap outside the image exists iff padding is used or the last window overhangs.
+  // (pad, avec and whether the k table applies select the loader variant, see F_*.)
   a.pad = (a.pH > 0 || a.pW > 0 || (a.Ho - 1) * a.sH + a.kH > a.H || (a.Wo - 1) * a.sW + a.kW > a.W) ? 1 : 0;
+  a.avec = p.mode == CV_FWD ? (a.K % 4 == 0) : p.mode == CV_WGRAD ? ((a.Ho * a.Wo) % 4 == 0) : 0;   // and aligned bases (set with the pointers)
   a.dKHW = make_fastdiv((uint32_t)khw);
   a.dKW = make_fastdiv((uint32_t)a.kW);
   a.dWo = make_fastdiv((uint32_t)a.Wo);
   a.dHoWo = make_fastdiv((uint32_t)(a.Ho * a.Wo));
-  a.dPhW = make_fastdiv((uint32_t)std::min(a.sW, a.W));
-  a.dCpg = make_fastdiv((uint32_t)std::max(1, a.CoutPG));
-  a.dTn = make_fastdiv((uint32_t)std::max(1, a.tiles_n));
-  a.dPh = make_fastdiv((uint32_t)a.phases);
+  a.dW = make_fastdiv((uint32_t)a.W);
+  a.dHW = make_fastdiv((uint32_t)(a.H * a.W));
+  a.dSH = make_fastdiv((uint32_t)a.sH);
+  a.dSW = make_fastdiv((uint32_t)a.sW);
+  a.dCpg = make_fastdiv((uint32_t)(p.mode == CV_FWD ? a.CinPG : a.CoutPG));
   return a;
 }
 
-// Loader flags of a launch.
+// Loader flags of a launch (avec must already account for the operand's alignment).
 inline int conv_flags(const ConvGemmArgs& a, int mode) {
-  if (a.kH > 32 || a.kW > 32) return F_WIDE | (mode == CV_DGRAD ? 0 : F_PAD);
-  if (mode == CV_DGRAD) return a.CoutPG % 8 == 0 ? F_TAP : 0;
-  int f = a.pad ? F_PAD : 0;
-  if (mode == CV_FWD) return f | (a.K % 4 == 0 ? F_AVEC : 0);
-  if (a.Ho * a.Wo % 4 == 0) f |= F_AVEC;
-  if (!a.pad && a.sW == 1 && a.Wo % 4 == 0) f |= F_BVEC;
+  // Tap-major order for the stride-1 input gradient only: measured on the CNN config it
+  // cuts the input gradient's index arithmetic (72.7 -> 63.8 us) but slows conv2d, whose
+  // k-contiguous weight rows then lose their vector loads and whose stages read 32
+  // channel planes instead of a few neighbouring rows (43.7 -> 68.9 us).
+  const bool tap = mode == CV_DGRAD && a.sH == 1 && a.sW == 1 && a.CoutPG % kCBK == 0;
+  if (tap) return F_TAP;
+  int f = 0;
+  if (a.avec && mode != CV_DGRAD) f |= F_AVEC;
+  if (a.pad && mode != CV_DGRAD) f |= F_PAD;
+  if ((mode == CV_FWD || mode == CV_DGRAD) && a.K <= kTab) f |= F_TAB;
   return f;
 }
 

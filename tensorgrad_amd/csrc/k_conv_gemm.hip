@@ -1,5 +1,5 @@
-// Implicit-GEMM convolution (NCHW, f32) on the gfx950 matrix cores (f32 products from
-// bf16 MFMAs, as x3_tile in gemm_dev.h). Nothing is materialised: each operand tile is gathered from
+// Implicit-GEMM convolution (NCHW, f32) on the gfx950 matrix cores
+// (v_mfma_f32_32x32x2_f32). Nothing is materialised: each operand tile is gathered from
 // the activations with the convolution's index map while it is staged into LDS.
 //
 // Per image b and group g (z = b * G + g), the three IR kinds are GEMMs
@@ -13,11 +13,16 @@
 // is split across blocks (deterministic: each split writes its own partial tile, a second
 // kernel adds the partials in split order).
 //
-// 256 threads make a 64 x 64 or 32 x 128 output tile in 32 x 32 wavefront tiles. Every
-// index is 32-bit (the host checks the sizes) and divisions by the geometry use precomputed
-// multiplicative inverses (FastDiv).
+// The tile machinery follows k_gemm (k_gemm.hip): 256 threads, 32 x 32 MFMA wave tiles,
+// k-permuted fragments (lane half h takes k = 4h .. 4h+3 of each group of 8), one fresh
+// accumulator per BK-k stage added to the running sum (blocked summation), double-buffered
+// LDS stages filled from registers prefetched during the previous stage's products.
+// A (the weight or dY operand) is staged k-contiguous, [row][BK + 4]; B is staged in the
+// direction its gather is contiguous: output positions (conv2d, input grad: consecutive
+// wo / wi) as [k][BN + 8], or k (weight grad: consecutive wo) as [n][BK + 4]. Every
+// index is 32-bit (the host checks that every tensor has fewer than 2^31 elements) and
+// divisions by the geometry use precomputed multiplicative inverses (FastDiv).
 #include "conv_gemm_dev.h"
-#include "gemm_dev.h"
 
 #include <algorithm>
 #include <stdexcept>
@@ -29,205 +34,178 @@ using namespace gd;
 using namespace cg;
 
 
-// An operand's ROWS x 16 stage in LDS: three planes of bf16, a row of 32 bytes each (XTile's layout).
-template <int ROWS>
-struct ConvStage {
-  static constexpr int PLANE = ROWS * 32, SIZE = 3 * PLANE;
-  template <int N>   // N k of a row, from k on: 4 or 8
-  __device__ __forceinline__ static void store(const float* q, char* L, int row, int k) {
-    uint32_t h[N / 2], m[N / 2], l[N / 2];
+// One operand's ROWS x BK stage in registers, as Tile in k_gemm.hip.
+template <int ROWS, bool KFAST>
+struct Stage {
+  static constexpr int LD = KFAST ? kCBK + 4 : ROWS + 8;
+  static constexpr int SIZE = KFAST ? ROWS * LD : kCBK * LD;
+  static constexpr int Q = ROWS * kCBK / (4 * kCT);
+  static_assert(Q >= 1, "tile too small for the block");
+  f32x4 q[Q];
+
+  __device__ __forceinline__ static void coords(int idx, int& rr, int& kk) {
+    if (KFAST) { rr = idx / (kCBK / 4); kk = (idx % (kCBK / 4)) * 4; }
+    else { rr = (idx % (ROWS / 4)) * 4; kk = idx / (ROWS / 4); }
+  }
+  __device__ __forceinline__ void store(float* L, int tid) const {
 #pragma unroll
-    for (int u = 0; u < N / 2; ++u) split3(q[2 * u], q[2 * u + 1], h[u], m[u], l[u]);
-    char* p = L + XTile<64, true>::at(row, k >> 3) + (k & 7) * 2;
-    put<N>(p, h);
-    put<N>(p + PLANE, m);
-    put<N>(p + 2 * PLANE, l);
+    for (int e = 0; e < Q; ++e) {
+      int rr, kk;
+      coords(tid + e * kCT, rr, kk);
+      if (KFAST) *reinterpret_cast<f32x4*>(L + rr * LD + kk) = q[e];
+      else *reinterpret_cast<f32x4*>(L + kk * LD + rr) = q[e];
+    }
   }
-  template <int N>
-  __device__ __forceinline__ static void put(char* p, const uint32_t* v) {
-    if constexpr (N == 8) *reinterpret_cast<u32x4*>(p) = (u32x4){v[0], v[1], v[2], v[3]};
-    else *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
-  }
-  __device__ __forceinline__ static bf16x8 frag(const char* L, int plane, int row, int h) {
-    return *reinterpret_cast<const bf16x8*>(L + plane * PLANE + XTile<64, true>::at(row, h));
+  __device__ __forceinline__ static f32x4 frag(const float* L, int row, int kb) {
+    if (KFAST) return *reinterpret_cast<const f32x4*>(L + row * LD + kb);
+    f32x4 v;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = L[(kb + u) * LD + row];
+    return v;
   }
 };
 
-// f32 products from six bf16 MFMAs, as x3_tile (gemm_dev.h, which gives the arithmetic and its error): the stage in one
-// half of the LDS is multiplied while the next is split into the other half and the third from here loaded. The terms of
-// four stages (KTab) are found at once by one wavefront.
-//
-// What bounds it: the vector port, and then the gathers. Per stage a wavefront of a 64 x 64 tile issues 6 MFMAs (which
-// keep the port for half their time) and about 95 vector instructions: 8 elements split (5.5 each), their offsets, the
-// running sum. An element is split once for each tap it meets. Tile: 4 blocks a CU hide each other's latencies; 64 x 128
-// was slower everywhere (its registers admit 3), and 32-row outputs take 128 columns so that A's share stays small.
-// [128, 32, 26, 26] * [64, 32, 3, 3]: forward 45 -> 32 us, input gradient 64 -> 44 us, weight gradient 50 -> 33 us
-// against f32 MFMAs; [32, 64, 33, 33] * [64, 64, 3, 3] with stride 2: 32 -> 23, 74 -> 23, 30 -> 25 us.
-template <int MODE, int BM, int BN, int F>
-__global__ __launch_bounds__(kCT, 4) void k_conv_gemm(ConvGemmArgs c) {
+// Pipeline: two register sets of staged loads, so the global loads of stage s + 2 are in
+// flight while stage s is multiplied and stage s + 1 waits in registers for its LDS slot.
+template <int MODE, bool FAST, int BM, int BN, int F>
+__global__ __launch_bounds__(kCT) void k_conv_gemm(ConvGemmArgs c) {
   constexpr int WGM = BM >= 64 ? 2 : 1, WGN = 4 / WGM;   // wave grid
-  constexpr int TN = BN / WGN / 32;                      // a wavefront's tiles: 32 x (TN * 32)
-  static_assert(BM / WGM == 32 && TN >= 1, "bad conv tile");
-  using LD = ConvLoader<MODE, BM, BN, F>;
-  using SA = ConvStage<BM>;
-  using SB = ConvStage<BN>;
-  __shared__ __attribute__((aligned(16))) char lds[2][SA::SIZE + SB::SIZE];
-  __shared__ __attribute__((aligned(16))) KTab tab[8];   // of stage s in tab[s % 8]
+  constexpr int WM = BM / WGM, WN = BN / WGN;            // wave tile
+  constexpr int TM = WM / 32, TN = WN / 32;
+  static_assert(TM >= 1 && TN >= 1 && WM % 32 == 0 && WN % 32 == 0, "bad conv tile");
+  using L = ConvLoader<MODE, FAST, BM, BN, F>;
+  using SA = Stage<BM, true>;
+  using SB = Stage<BN, L::BKF>;
+  static_assert(SA::Q == L::QA && SB::Q == L::QB, "stage / loader mismatch");
+  constexpr bool TAB = (F & F_TAB) != 0;
+  __shared__ __attribute__((aligned(16))) float As[2][SA::SIZE];
+  __shared__ __attribute__((aligned(16))) float Bs[2][SB::SIZE];
+  __shared__ uint32_t ktab[TAB ? 2 * kTab : 2];
 
-  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int wm0 = (wave / WGN) * 32, wn0 = (wave % WGN) * TN * 32;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int wm0 = (wave / WGN) * WM, wn0 = (wave % WGN) * WN;
+  L ld;
+  ld.init(c, block_pos<BM, BN>(c, blockIdx.x, gridDim.x, MODE), tid);
+  const int kbeg = ld.bp.kbeg, kend = ld.bp.kend;
+  if (TAB) {
+    for (int k = tid; k < c.K; k += kCT) k_term(c, MODE, k, ktab[2 * k], ktab[2 * k + 1]);
+    __syncthreads();
+  }
+
+  SA sa[2];
+  SB sb[2];
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
   const int lrow = lane % 32, h = lane / 32;
-  const bool has_a = BM == 64 || wave < 2;
-  ConvMap<MODE, F> map;
-  map.template init<BM, BN>(c, blockIdx.x, gridDim.x);
-  if (MODE == CV_DGRAD && map.n0 >= map.N) return;       // a smaller phase than the first
-  auto put_terms = [&](int st) {   // of four stages
-    const int s = st + lane / kCBK, l = lane % kCBK;
-    const KTerm t = map.k_term(c, map.kbeg + s * kCBK + l);
-    KTab& k = tab[s & 7];
-    k.a[l] = t.a;
-    k.b[l] = t.b;
-    k.t0[l] = t.t0;
-    k.t1[l] = t.t1;
-  };
-  if (wave == 0) put_terms(0);
-  LD ld;
-  ld.init(map, c, tid);
-  __syncthreads();
-
-  float qa[2][4], qb[2][LD::PB];
-  f32x16 acc[TN], part[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = part[j][r] = 0.0f;
-  auto load = [&](int st, int set) { ld.load(map, c, tab[st & 7], has_a, qa[set], qb[set]); };
-  auto store = [&](int set, float sign) {
-    if (has_a) {
-      float q[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = sign * qa[set][u];
-      SA::template store<4>(q, lds[set], LD::a_row(tid), ld.ka);
-    }
-#pragma unroll
-    for (int e = 0; e < LD::NR; ++e)
-      SB::template store<LD::PB / LD::NR>(qb[set] + e * (LD::PB / LD::NR), lds[set] + SA::SIZE, LD::b_row(tid, e), ld.kb);
-  };
-  auto meet = [&]() {   // LDS traffic only: the loads of later stages stay in flight
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  const int nst = map.kbeg < map.kend ? (map.kend - map.kbeg + kCBK - 1) / kCBK : 0;
-  // Stages past the last read as zeros (their terms are masked), so nothing here tests for the end.
-  // Every two stages begin a new part, and the running sums take the last. The bf16 MFMAs round towards one side by a
-  // little (2^-27 of a part), which over many parts of either sign would be all of the error; so every other part is
-  // made of negated A, and the running sums change sign each time: the weight gradient's error over K = 73728 is 1.5e-7 so, 3.9e-7 without.
-  auto sign = [](int st) { return (st & 2) ? -1.0f : 1.0f; };
-  auto body = [&](int st, auto ptag) {
-    constexpr int P = decltype(ptag)::value;
-    constexpr bool FRESH = P == 0;
-    if (P == 0 && (st & 15) == (wave << 2)) put_terms(st + 4);
-    const char *La = lds[P], *Lb = La + SA::SIZE;
-    constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};   // small terms first
-    bf16x8 a[3], b[TN][3];
-#pragma unroll
-    for (int o = 0; o < 3; ++o) {
-      a[o] = SA::frag(La, o, wm0 + lrow, h);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) b[j][o] = SB::frag(Lb, o, wn0 + j * 32 + lrow, h);
-    }
-    store(P ^ 1, sign(st + 1));
-    load(st + 3, P ^ 1);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      if (FRESH) acc[j] = part[j] - acc[j];
-#pragma unroll
-      for (int t = 0; t < 6; ++t) {
-        const f32x16 p = FRESH && t == 0 ? (f32x16)(0.0f) : part[j];
-        part[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t]], b[j][PB[t]], p, 0, 0, 0);
-      }
-    }
-    meet();
-  };
+  const int nst = kbeg < kend ? (kend - kbeg + kCBK - 1) / kCBK : 0;
   if (nst > 0) {
-    load(0, 0);
-    load(1, 1);
-    store(0, 1.0f);
-    load(2, 0);
+    ld.load(c, kbeg, sa[0].q, sb[0].q, ktab);
+    if (nst > 1) ld.load(c, kbeg + kCBK, sa[1].q, sb[1].q, ktab);
+    sa[0].store(As[0], tid);
+    sb[0].store(Bs[0], tid);
   }
-  meet();
-  for (int st = 0; st < nst; st += 2) {
-    body(st, IntTag<0>{});
-    if (st + 1 < nst) body(st + 1, IntTag<1>{});
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = sign(nst - 1) * (part[j][r] - acc[j][r]);
-
-  // Values that are not finite do not split (x3_tile): such a wavefront multiplies its tile again with f32 MFMAs.
-  float bad = 0.0f;   // 0 * v is 0 for a finite v and NaN otherwise
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) bad = fmaf(acc[j][r], 0.0f, bad);
-  if (__builtin_amdgcn_ballot_w64(bad != 0.0f) != 0) {
-    const uint32_t ar = map.a_row(c, map.m0 + wm0 + lrow);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const BTerm br = map.b_row(c, map.n0 + wn0 + j * 32 + lrow);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
-      for (int kb = map.kbeg; kb < map.kend; kb += 32) {
-        f32x16 sum = (f32x16)(0.0f);
-#pragma unroll 1
-        for (int u = 0; u < 32; u += 2) {
-          const KTerm t = map.k_term(c, kb + u + h);
-          const float av = ldb(map.sa, ar + t.a);
-          const float bv = ldb(map.sb, (br.off + t.b) | map.outside(c, br.t0, br.t1, t.t0, t.t1));
-          sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, sum, 0, 0, 0);
-        }
-        acc[j] += sum;
-      }
+  __syncthreads();
+  for (int st = 0; st < nst; ++st) {
+    const int cur = st & 1;
+    // registers of stage st were stored at the previous iteration: refill them with st + 2
+    if (st + 2 < nst) {
+      if (cur == 0) ld.load(c, kbeg + (st + 2) * kCBK, sa[0].q, sb[0].q, ktab);
+      else ld.load(c, kbeg + (st + 2) * kCBK, sa[1].q, sb[1].q, ktab);
     }
+    const float* Ac = As[cur];
+    const float* Bc = Bs[cur];
+    // Blocked accumulation: a fresh partial sum per stage, added to the running total.
+    f32x16 part[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[i][j][r] = 0.0f;
+#pragma unroll
+    for (int grp = 0; grp < kCBK / 8; ++grp) {
+      const int kb = grp * 8 + h * 4;
+      f32x4 av[TM], bv[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) av[i] = SA::frag(Ac, wm0 + i * 32 + lrow, kb);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bv[j] = SB::frag(Bc, wn0 + j * 32 + lrow, kb);
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][jj], bv[j][jj], part[i][j], 0, 0, 0);
+    }
+    if (st + 1 < nst) {
+      if (cur == 0) { sa[1].store(As[1], tid); sb[1].store(Bs[1], tid); }
+      else { sa[0].store(As[0], tid); sb[0].store(Bs[0], tid); }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += part[i][j];
+    __syncthreads();
   }
 
   // Register r of lane l holds row (r/4)*8 + (l/32)*4 + r%4, column l%32.
   float* O = (MODE == CV_WGRAD && c.splits > 1) ? c.work : c.out;
-  const int64_t rs = map.out_rs(c);
-  const bool epi = MODE != CV_WGRAD && c.epi != kConvEpiNone;
+  const int64_t rs = ld.out_rs(c);
+  if (MODE != CV_WGRAD && c.epi != kConvEpiNone) {
+    // The layer's pointwise step at the store (one group, G = 1: channel gm). Every bias /
+    // mask value of the wavefront's outputs is loaded first (clamped in range): loaded
+    // between the stores, each would wait for the stores before it.
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int gn = min(ld.bp.n0 + wn0 + j * 32 + lrow, c.N - 1);
+      const int64_t cofs = ld.out_col(c, gn);
+      float e[TM][16];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int gm = min(ld.bp.m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4), c.M - 1);
+          e[i][r] = c.epi == kConvEpiBiasRelu ? c.ebias[gm] : c.emask[cofs + gm * rs];
+        }
+      if (ld.bp.n0 + wn0 + j * 32 + lrow >= c.N) continue;
+      float* col = O + cofs;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int gm = ld.bp.m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
+          if (gm >= c.M) continue;
+          float v = acc[i][j][r];
+          if (c.epi == kConvEpiBiasRelu) {
+            const float a = v + e[i][r];
+            v = a != a ? __uint_as_float(0x7fc00000u) : (a > 0.0f ? a : 0.0f);
+          } else {
+            v = e[i][r] > 0.0f ? v : 0.0f;
+          }
+          col[gm * rs] = v;
+        }
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int gn = map.n0 + wn0 + j * 32 + lrow;
-    const int64_t cofs = map.out_col(c, min(gn, map.N - 1));
-    float e[16];
-    if (epi) {
-      // The layer's pointwise step at the store (one group, G = 1: channel gm). Every bias / mask value is loaded first
-      // (clamped in range): loaded between the stores, each would wait for the stores before it.
+    const int gn = ld.bp.n0 + wn0 + j * 32 + lrow;
+    if (gn >= c.N) continue;
+    float* col = O + ld.out_col(c, gn);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int gm = min(map.m0 + wm0 + (r / 4) * 8 + h * 4 + (r % 4), c.M - 1);
-        e[r] = c.epi == kConvEpiBiasRelu ? c.ebias[gm] : c.emask[cofs + gm * rs];
+        const int gm = ld.bp.m0 + wm0 + i * 32 + (r / 4) * 8 + h * 4 + (r % 4);
+        if (gm < c.M) col[gm * rs] = acc[i][j][r];
       }
-    }
-    if (gn >= map.N) continue;
-    float* col = O + cofs;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int gm = map.m0 + wm0 + (r / 4) * 8 + h * 4 + (r % 4);
-      if (gm >= c.M) continue;
-      float v = acc[j][r];
-      if (epi) {
-        if (c.epi == kConvEpiBiasRelu) {
-          const float a = v + e[r];
-          v = a != a ? __uint_as_float(0x7fc00000u) : (a > 0.0f ? a : 0.0f);
-        } else {
-          v = e[r] > 0.0f ? v : 0.0f;
-        }
-      }
-      col[gm * rs] = v;
-    }
   }
 }
 
@@ -422,33 +400,44 @@ bool small_wgrad_ok(const ConvDesc& d) {
   return taps <= kSmallTaps && d.B * d.Cout * taps * 4 <= kConvWorkBytes;
 }
 
-template <int MODE, int F>
+template <int MODE, bool FAST, int F>
 void launch_tile(const ConvPlan& p, const ConvGemmArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)p.blocks);
-  if (p.bm == 32) klaunch(k_conv_gemm<MODE, 32, 128, F>, grid, kCT, 0, st, a);
-  else klaunch(k_conv_gemm<MODE, 64, 64, F>, grid, kCT, 0, st, a);
+  if (p.bm == 32) klaunch(k_conv_gemm<MODE, FAST, 32, 128, F>, grid, kCT, 0, st, a);
+  else if (p.bn == 64) klaunch(k_conv_gemm<MODE, FAST, 64, 64, F>, grid, kCT, 0, st, a);
+  else klaunch(k_conv_gemm<MODE, FAST, 64, 128, F>, grid, kCT, 0, st, a);
 }
 
 // The loader variant (conv_flags) of a launch picks the instantiation.
 template <int MODE>
-void launch_mode(const ConvPlan& p, const ConvGemmArgs& a, hipStream_t st) {
+void launch_mode(const ConvPlan& p, const ConvGemmArgs& a, bool fast, hipStream_t st) {
   const int f = conv_flags(a, MODE);
-  if constexpr (MODE == CV_DGRAD) {
-    switch (f) {
-      case F_WIDE: return launch_tile<MODE, F_WIDE>(p, a, st);
-      case F_TAP: return launch_tile<MODE, F_TAP>(p, a, st);
-      default: return launch_tile<MODE, 0>(p, a, st);
+  if (MODE == CV_DGRAD && fast && (f & F_TAP)) return launch_tile<MODE, true, F_TAP>(p, a, st);
+  if (MODE == CV_FWD && (f & F_TAP)) {
+    if (f & F_PAD) launch_tile<MODE, true, F_TAP | F_PAD>(p, a, st);
+    else launch_tile<MODE, true, F_TAP>(p, a, st);
+    return;
+  }
+  if (MODE == CV_DGRAD) {
+    if (!fast) launch_tile<MODE, false, 0>(p, a, st);
+    else if (f & F_TAB) launch_tile<MODE, true, F_TAB>(p, a, st);
+    else launch_tile<MODE, true, 0>(p, a, st);
+    return;
+  }
+  const int fa = f & (F_AVEC | F_PAD);
+  if (MODE == CV_FWD && (f & F_TAB)) {
+    switch (fa) {
+      case 0: launch_tile<MODE, true, F_TAB>(p, a, st); return;
+      case F_AVEC: launch_tile<MODE, true, F_TAB | F_AVEC>(p, a, st); return;
+      case F_PAD: launch_tile<MODE, true, F_TAB | F_PAD>(p, a, st); return;
+      default: launch_tile<MODE, true, F_TAB | F_AVEC | F_PAD>(p, a, st); return;
     }
-  } else {
-    switch (f) {
-      case F_WIDE | F_PAD: return launch_tile<MODE, F_WIDE | F_PAD>(p, a, st);
-      case F_AVEC: return launch_tile<MODE, F_AVEC>(p, a, st);
-      case F_PAD: return launch_tile<MODE, F_PAD>(p, a, st);
-      case F_AVEC | F_PAD: return launch_tile<MODE, F_AVEC | F_PAD>(p, a, st);
-      case F_AVEC | F_BVEC:
-        if constexpr (MODE == CV_WGRAD) return launch_tile<MODE, F_AVEC | F_BVEC>(p, a, st);
-      default: return launch_tile<MODE, 0>(p, a, st);
-    }
+  }
+  switch (fa) {
+    case 0: launch_tile<MODE, true, 0>(p, a, st); return;
+    case F_AVEC: launch_tile<MODE, true, F_AVEC>(p, a, st); return;
+    case F_PAD: launch_tile<MODE, true, F_PAD>(p, a, st); return;
+    default: launch_tile<MODE, true, F_AVEC | F_PAD>(p, a, st); return;
   }
 }
 
@@ -472,13 +461,14 @@ void conv2d_gemm(const float* x, const float* w, float* y, const ConvDesc& d, hi
     a.epi = kConvEpiBiasRelu;
     a.ebias = bias;
   }
+  a.avec = a.avec && ((uintptr_t)w & 15) == 0;
   if (d.CinPG * d.kH * d.kW <= kSmallTaps && (d.Cout / d.G) * kSmallTaps <= kSmallW) {
     // the K taps of a row of W are contiguous: W[co][cl][kh][kw] = w[co * K + q]
     const int64_t n = d.B * d.G * ((d.Ho * d.Wo + 255) / 256);
     if (n > 0) klaunch(k_conv_small_fwd, (unsigned)n, 256, 0, st, a);
     return;
   }
-  if (p.blocks > 0) launch_mode<CV_FWD>(p, a, st);
+  if (p.blocks > 0) launch_mode<CV_FWD>(p, a, true, st);
 }
 
 void conv2d_input_grad_gemm(const float* w, const float* dy, float* dx, const ConvDesc& d, hipStream_t st,
@@ -490,7 +480,7 @@ void conv2d_input_grad_gemm(const float* w, const float* dy, float* dx, const Co
     a.epi = kConvEpiReluMask;
     a.emask = mask;
   }
-  if (p.blocks > 0) launch_mode<CV_DGRAD>(p, a, st);
+  if (p.blocks > 0) launch_mode<CV_DGRAD>(p, a, d.sH == 1 && d.sW == 1, st);
 }
 
 void conv2d_weight_grad_gemm(const float* x, const float* dy, float* dw, const ConvDesc& d, float* work,
@@ -498,6 +488,7 @@ void conv2d_weight_grad_gemm(const float* x, const float* dy, float* dw, const C
   const ConvPlan p = conv_plan(CV_WGRAD, d);
   ConvGemmArgs a = make_args(d, p);
   a.x = x; a.dy = dy; a.out = dw; a.work = work;
+  a.avec = a.avec && ((uintptr_t)dy & 15) == 0;
   if (small_wgrad_ok(d)) {
     if (!work) throw std::runtime_error("conv2d_weight_grad: missing workspace");
     if (d.B <= 0 || d.Cout <= 0) return;
@@ -518,7 +509,7 @@ void conv2d_weight_grad_gemm(const float* x, const float* dy, float* dw, const C
   }
   if (p.blocks <= 0) return;
   if (p.splits > 1 && !work) throw std::runtime_error("conv2d_weight_grad: missing workspace");
-  launch_mode<CV_WGRAD>(p, a, st);
+  launch_mode<CV_WGRAD>(p, a, true, st);
   if (p.splits > 1) {
     const int64_t per = (int64_t)a.G * a.M * a.N;
     if (per < 16384 && p.splits > 16) {

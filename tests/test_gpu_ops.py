@@ -909,37 +909,6 @@ def test_conv_kernels(impl, case):
             os.environ['TG_CONV'] = old
 
 
-@pytest.mark.parametrize('B,Ci,H,W,Co,G,kh,kw,s,pd', [
-    (3, 16, 13, 11, 33, 1, 3, 3, 3, 1),     # input gradient: 9 phases of unequal size, channels no multiple of 8
-    (2, 32, 12, 12, 64, 1, 2, 2, 3, 0),     # phases that no tap reaches
-    (2, 24, 17, 19, 72, 1, 5, 3, 2, 2),     # phases of 6 to 2 taps
-    (1, 3, 40, 70, 65, 1, 3, 35, 1, 1),     # more than 32 columns of taps
-    (7, 17, 10, 12, 31, 1, 3, 3, 1, 0),     # odd channels; K = 153
-    (5, 48, 9, 16, 48, 2, 3, 3, 20, 1),     # stride past the image: one position per phase
-])
-def test_conv_split_tile(B, Ci, H, W, Co, G, kh, kw, s, pd):
-    """The convolutions' loaders at the edges of their forms, and infinities: an infinite input reaches the outputs that
-    read it and no other. Tolerance as of the products (32 k and 16 k roundings of at most 2^-24 each)."""
-    Ho, Wo = (H + 2 * pd - kh) // s + 1, (W + 2 * pd - kw) // s + 1
-    x, w, dy = _rand([B, Ci, H, W], 41), _rand([Co, Ci // G, kh, kw], 42), _rand([B, Co, Ho, Wo], 43)
-
-    def check(*kinds):
-        for body, names in kinds:
-            got, want = run_both(body, {n: {'x': x, 'w': w, 'd': dy}[n] for n in names})
-            assert np.array_equal(np.isfinite(got), np.isfinite(want))
-            ok = np.isfinite(want)
-            gemm_close(got[ok], want[ok])
-    xi, wi, di = (lambda: tensor_input('x', list(x.shape))), (lambda: tensor_input('w', list(w.shape))), \
-        (lambda: tensor_input('d', list(dy.shape)))
-    fwd = lambda: O.conv2d(xi(), wi(), stride=s, padding=pd, groups=G)
-    dgrad = lambda: O.conv2d_input_grad(wi(), di(), H, W, s, s, pd, pd, G)
-    wgrad = lambda: O.conv2d_weight_grad(xi(), di(), kh, kw, s, s, pd, pd, G)
-    check((fwd, 'xw'), (dgrad, 'wd'), (wgrad, 'xd'))
-    x[0, Ci // 2, H // 2, W // 2] = np.inf
-    dy[B - 1, Co - 1, Ho - 1, 0] = np.inf
-    check((fwd, 'xw'), (dgrad, 'wd'))
-
-
 @pytest.mark.parametrize('B,Ci,H,Co,k,pd', [(4, 3, 12, 16, 3, 1), (8, 1, 28, 32, 3, 0), (2, 8, 9, 40, 5, 2)])
 def test_conv_epilogues(B, Ci, H, Co, k, pd):
     """A convolution whose output only its layer's pointwise step reads applies that step
