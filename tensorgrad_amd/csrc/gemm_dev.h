@@ -795,10 +795,12 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
     if (st + 1 < cnt) body(st + 1, IntTag<1>{}, IntTag<0>{});
     else meet();
   }
+  // The last part and the running sums have opposite signs. Adding +0.0 makes a sum of zeros +0.0 where the sign is -1.
+  const float last = sign(cnt - 1);
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = (part[i][j] - acc[i][j]) * sign(cnt - 1);   // (by element: spills)
+    for (int j = 0; j < TN; ++j) acc[i][j] = (part[i][j] - acc[i][j]) * last + 0.0f;   // (by element: spills)
   if (KG > 1) {
     float* X = reinterpret_cast<float*>(lds);   // every group has passed its last read of the buffers
     if (kg > 0) {

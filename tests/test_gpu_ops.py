@@ -741,6 +741,27 @@ def test_matmul_split_tile_infinities(M, N, K):
     gemm_close(got[20][ok[20]], want[20][ok[20]])
 
 
+@pytest.mark.parametrize('M,N,K', [(64, 64, 32), (128, 192, 48), (128, 192, 64), (96, 130, 97), (128, 192, 512),
+                                   (256, 256, 2048)])
+def test_matmul_split_tile_zeros_are_positive(M, N, K):
+    """A sum of zeros is +0.0 at every number of stages, as the oracle's is: -0.0 would turn a reciprocal or a reciprocal
+    square root of it from +inf to -inf. Zero rows, zero columns and negative partners."""
+    a, b = _rand([M, K], 149), _rand([N, K], 150)
+    a[3], a[M - 1], b[5], b[N - 1] = 0, -0.0, 0, -0.0
+    ins = {'a': a, 'b': b}
+
+    def product():
+        return O.matmul(tensor_input('a', [M, K]), O.swap_axes(tensor_input('b', [N, K]), -1, -2))
+    got, want = run_both(product, ins)
+    zero = np.zeros((M, N), bool)
+    zero[[3, M - 1]] = zero[:, [5, N - 1]] = True
+    assert np.all(want[zero] == 0) and not np.signbit(want[zero]).any()
+    assert np.all(got[zero] == 0) and not np.signbit(got[zero]).any()
+    for inverse in (lambda x: O.div(1.0, x), O.rsqrt):
+        got, want = run_both(lambda: inverse(product()), ins)
+        assert np.all(got[zero] == np.inf) and np.all(want[zero] == np.inf)
+
+
 def test_matmul_split_tile_batched_and_summed():
     """Batched head views (two batch strides), and a sum of products whose segments hold an infinity."""
     B, T, H, d = 3, 100, 2, 80
