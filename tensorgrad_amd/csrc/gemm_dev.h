@@ -537,11 +537,16 @@ struct StoreC {   // (tile_finish stores it)
 // The bf16 MFMAs run at 16 times the f32 rate. An f32 value is exactly the sum of three bf16 values (round to nearest,
 // then the same of what is left, twice: 8 + 8 + 8 bits), so a product is nine bf16 products, of which the three below
 // 2^-25 of the largest (mid * low, low * mid, low * low) are left out: six MFMAs in place of sixteen's worth of time.
-// Accuracy against 64 bits is no worse than the f32 tile's (norm-wise, K = 512 .. 4096: 0.9e-7 .. 1.3e-7 against
-// 1.1e-7 .. 1.8e-7): the products are exact, an MFMA adds 16 of them with one rounding where the f32 one adds two, and
-// every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum.
+// Operands are scaled by 2^16 on the way, which puts the last bit of the smallest f32 (2^-149) on bf16's (2^-133): without
+// it the low terms of values below 2^-110 would be lost (2^-120: wrong by 2e-5). The sums are scaled back by 2^-32.
+// Accuracy against 64 bits is no worse than the f32 tile's over sums of many terms (norm-wise, K = 64 .. 4096: 0.7e-7 ..
+// 1.1e-7 against 1.4e-7 .. 1.7e-7; values of one sign 0.5e-7 .. 0.6e-7 against 1.1e-7 .. 0.5e-7): an MFMA adds 16 exact
+// bf16 products with one rounding where the f32 one adds two, and every 32 k go into a fresh accumulator (the small terms
+// first) that is added to the running sum. A sum that one of its terms makes up has that term's error, the products left
+// out and the MFMA's rounding: up to 1.4 units in the last place (0.39 rms), where an f32 product rounds once (0.5, 0.29).
 // Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
-// are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile.
+// are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile; so
+// do values and sums that the scale takes past the f32 range (2^112 and 2^96).
 //
 // What bounds it: per 16 k a wavefront with a 64 x 64 tile issues 24 MFMAs (32 cycles each) and about 130 vector
 // instructions (5.5 per element split, 2 per accumulator), and an MFMA keeps the vector port for half its time, so the
@@ -576,6 +581,7 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& h, uint32_t
 }
 
 constexpr int kXK = 16;   // k of a stage: one MFMA's
+constexpr float kXScale = 65536.0f;   // of an operand on its way to LDS
 
 // One operand's ROWS x 16 stage for 256 threads. In LDS a plane is rows of 32 bytes whose two 16-byte chunks (8 k each)
 // are swapped by a function of the row, so the fragment reads (a lane's 8 k of its row) meet no bank twice; rows of a
@@ -631,8 +637,7 @@ struct XTile {
     if (n == 2) *reinterpret_cast<u32x2*>(p) = (u32x2){v[0], v[1]};
     else *reinterpret_cast<uint32_t*>(p) = v[0];
   }
-  template <bool SIGNED>   // SIGNED: times sign (1 or -1)
-  __device__ __forceinline__ static void store(const float* q, char* L, int tid, float sign) {
+  __device__ __forceinline__ static void store(const float* q, char* L, int tid, float scale) {
     constexpr int W = KFAST ? 2 : PK / 2;          // pairs of k in a unit
     constexpr int UNITS = KFAST ? PER / 4 : 2;
 #pragma unroll
@@ -642,8 +647,7 @@ struct XTile {
       uint32_t h[W], m[W], l[W];
 #pragma unroll
       for (int u = 0; u < W; ++u) {
-        const float x0 = q[(e * W + u) * 2], x1 = q[(e * W + u) * 2 + 1];
-        split3(SIGNED ? sign * x0 : x0, SIGNED ? sign * x1 : x1, h[u], m[u], l[u]);
+        split3(scale * q[(e * W + u) * 2], scale * q[(e * W + u) * 2 + 1], h[u], m[u], l[u]);
       }
       char* p = L + at(row, k >> 3) + (k & 7) * 2;
       put(p, h, W);
@@ -757,8 +761,8 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
     for (int j = 1; j < TN; ++j)
 #pragma unroll
       for (int o = 0; o < 3; ++o) bb[OB[o]][j] = TB::frag(Lb, OB[o], wn0 + j * 32 + lrow, h);
-    TA::template store<SIGNA>(qa[P ^ 1], mine + (P ^ 1) * BUF, tid, sign(st + 1));
-    TB::template store<!SIGNA>(qb[P ^ 1], mine + (P ^ 1) * BUF + TA::SIZE, tid, sign(st + 1));
+    TA::store(qa[P ^ 1], mine + (P ^ 1) * BUF, tid, SIGNA ? sign(st + 1) * kXScale : kXScale);
+    TB::store(qb[P ^ 1], mine + (P ^ 1) * BUF + TA::SIZE, tid, SIGNA ? kXScale : sign(st + 1) * kXScale);
     ahead(st + 3, P ^ 1);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -783,8 +787,8 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
       TB::mask(qb[0], keep, tid);
     }
     ahead(1, 1);
-    TA::template store<false>(qa[0], mine, tid, 1.0f);
-    TB::template store<false>(qb[0], mine + TA::SIZE, tid, 1.0f);
+    TA::store(qa[0], mine, tid, kXScale);
+    TB::store(qb[0], mine + TA::SIZE, tid, kXScale);
     ahead(2, 0);
   }
   meet();
@@ -796,7 +800,7 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
     else meet();
   }
   // The last part and the running sums have opposite signs. Adding +0.0 makes a sum of zeros +0.0 where the sign is -1.
-  const float last = sign(cnt - 1);
+  const float last = sign(cnt - 1) / (kXScale * kXScale);
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll

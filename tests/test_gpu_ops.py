@@ -762,6 +762,22 @@ def test_matmul_split_tile_zeros_are_positive(M, N, K):
         assert np.all(got[zero] == np.inf) and np.all(want[zero] == np.inf)
 
 
+@pytest.mark.parametrize('e', [-100, -112, -120, -126, -135, -149])
+def test_matmul_split_tile_small_operands(e):
+    """Operands down to the smallest f32 against ones that bring the product back to ordinary size, on either side: the
+    same tolerance as for ordinary values (the f32 product of such values has no larger error either). At 2^-149 times
+    2^80 the products are near 2^-69, still ordinary."""
+    M, N, K = 128, 192, 256
+    r = np.random.default_rng(151)
+    a = (r.uniform(1, 2, (M, K)) * r.choice([-1, 1], (M, K)) * 2.0 ** e).astype(np.float32)
+    assert np.any(a)
+    for up in (80, 120):   # (2^120 leaves the scaled operands' range: those tiles are multiplied again in f32)
+        b = (r.uniform(-1, 1, (N, K)) * 2.0 ** min(-e, up)).astype(np.float32)
+        for m, n, x, y in ((M, N, a, b), (N, M, b, a)):
+            got, want = run_both(_product(m, n, K, False, True), {'a': x, 'b': y})
+            gemm_close(got * 2.0 ** 40, want.astype(np.float64) * 2.0 ** 40)
+
+
 def test_matmul_split_tile_batched_and_summed():
     """Batched head views (two batch strides), and a sum of products whose segments hold an infinity."""
     B, T, H, d = 3, 100, 2, 80
