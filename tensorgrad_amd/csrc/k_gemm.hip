@@ -282,22 +282,23 @@ __global__ __launch_bounds__(256 * KG, x3_waves(BM, BN)) void k_gemm_x3_group(co
   x3_tile<BM, BN, AK, BKF, KG, StoreC>(g, b - starts[p], StoreC{});
 }
 
-// Sum split-K partials in split order into C (eight partial loads in flight per thread).
+// Sum split-K partials in split order into C (eight partial loads in flight per thread). In f64: 61 partials of a sum of
+// one sign added in f32 were most of its error ([256, 65536] x [65536, 256]: 1.06e-7 against 64 bits, so 2.8e-8), and the
+// launch is bound by its loads.
 __global__ void k_splitk_reduce(const float* __restrict__ work, int splits, int64_t sOs, GemmDesc d) {
   const int64_t MN = d.M * d.N, total = MN * d.batch;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    float s = 0.0f;
+    double s = 0.0;
     for (int sp0 = 0; sp0 < splits; sp0 += 8) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = sp0 + u < splits ? work[(sp0 + u) * sOs + i] : 0.0f;
+      for (int u = 0; u < 8; ++u) v[u] = work[min(sp0 + u, splits - 1) * sOs + i];   // (without a branch: back to back)
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (sp0 + u < splits) s += v[u];
+      for (int u = 0; u < 8; ++u) s += sp0 + u < splits ? (double)v[u] : 0.0;
     }
     const int64_t zz = i / MN, r = i % MN, m = r / d.N, n = r % d.N;
     const int64_t z0 = zz / d.bdiv, z1 = zz % d.bdiv;
-    d.C[z0 * d.sCz0 + z1 * d.sCz1 + m * d.sCm + n * d.sCn] = s;
+    d.C[z0 * d.sCz0 + z1 * d.sCz1 + m * d.sCm + n * d.sCn] = (float)s;
   }
 }
 

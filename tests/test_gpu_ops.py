@@ -778,6 +778,16 @@ def test_matmul_split_tile_small_operands(e):
             gemm_close(got * 2.0 ** 40, want.astype(np.float64) * 2.0 ** 40)
 
 
+@pytest.mark.parametrize('M,N,K', [(256, 256, 16384), (130, 260, 20000), (64, 64, 32768), (300, 100, 40000)])
+def test_matmul_long_sums_of_one_sign(M, N, K):
+    """Sums of thousands of positive terms, split over K: the partials are added in f64, so what is left is the partials'
+    own rounding, which averages out over them, and the result's, at most 2^-24 of it (in f32 the additions of 32 and
+    more partials alone came to 5e-8 to 1e-7)."""
+    a, b = _rand([M, K], 152, 0, 1), _rand([K, N], 153, 0, 1)
+    got, want = run_both(_product(M, N, K, False, False), {'a': a, 'b': b})
+    gemm_close(got, want, 2.0 ** -24)
+
+
 def test_matmul_split_tile_batched_and_summed():
     """Batched head views (two batch strides), and a sum of products whose segments hold an infinity."""
     B, T, H, d = 3, 100, 2, 80
