@@ -407,16 +407,19 @@ XPlan x3_plan(const GemmDesc& d) {
   return best;
 }
 
-// One tiling for several unsplit products in one launch; its time in us.
+// One tiling for several unsplit products in one launch; its time in us, 1e30 where a sum would be longer than the error of
+// the f32 launches they replace allows.
 int x3_group_tiling(const GemmDesc* ds, int n, double* us_out) {
-  int best = -1;
-  double best_us = 0.0;
-  // Together these fill the chip with 64 x 64 tiles of one running sum over all of K: the f32 tiles' error then has
-  // variance 1.1 + 0.97e-3 k (x3_range), which allows longer ranges.
+  int best = kXTilingCount - 1;   // (64 x 64 by four groups: takes any)
+  double best_us = 1e30;
+  // The f32 launches: below 512 tiles of 64 x 64 split products, whose f32 sum adds 0.05e-14 or more a split to the variance
+  // (x3_range): [256, 64] over K = 8192 1.84e-7 in 32 splits, 1.68e-7 here in sums of 2048. From 512 tiles on a group that
+  // fills the chip, one running sum over all of K: 1.1 + 0.97e-3 k.
   int64_t t64 = 0;
   for (int q = 0; q < n; ++q) t64 += (ds[q].M + 63) / 64 * ((ds[q].N + 63) / 64) * ds[q].batch;
   auto range = [&](const GemmDesc& d) {
-    return t64 >= 512 && d.K > kShortK ? std::max(x3_range(d), 512 + (int64_t)(0.75 * (double)d.K)) : x3_range(d);
+    const int64_t split = x3_range(d) + 45 * std::min(plan_for(d).splits, 48);
+    return t64 >= 512 && d.K > kShortK ? std::max(split, 512 + (int64_t)(0.75 * (double)d.K)) : split;
   };
   for (int t = 0; t < kXTilingCount; ++t) {
     const XTiling& x = kXTilings[t];
@@ -428,10 +431,10 @@ int x3_group_tiling(const GemmDesc* ds, int n, double* us_out) {
       work += x3_tiles(x, ds[q]) * ds[q].K;
       kmax = std::max(kmax, ds[q].K);
     }
-    if (!fits && !(x.bm == 64 && x.bn == 64 && x.kg == 4)) continue;   // (the one that takes them all)
+    if (!fits) continue;
     // the launch ends with its longest tile; short ones fill in beside it
     const double us = std::max(x3_time(x, 1, 1, kmax), x3_time(x, tiles, 1, (work + tiles - 1) / tiles));
-    if (best < 0 || us < best_us) { best = t; best_us = us; }
+    if (us < best_us) { best = t; best_us = us; }
   }
   if (us_out) *us_out = best_us;
   return best;

@@ -7,8 +7,10 @@ import re
 
 import pytest
 
-from tensorgrad_amd import backend, configs
+from tensorgrad_amd import backend, configs, nn
+from tensorgrad_amd import ops as O
 from tensorgrad_amd.build_ir import build_forward_ir, build_training_ir
+from tensorgrad_amd.module import Module
 
 HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), 'include', 'tg.h')
 
@@ -318,6 +320,30 @@ def test_bias_sums_from_partials_alone_run_every_step():
     nodes = backend.plan(ir.wire_json())['nodes']
     sums = [n for n in nodes if n['kind'] == 'reduce' and n['shape'] == '3 column sums']
     assert len(sums) == 1 and sums[0]['ops'] == 'sum_partials,sum_partials,sum_partials'
+
+
+def _weight_gradients(rows, count, d_in, d_out):
+    """A step whose `count` weight gradients are products [d_in, rows] x [rows, d_out] of the same kind."""
+    class Layers(Module):
+        def __init__(self):
+            self.w = [nn.Linear(d_in, d_out, bias=False) for _ in range(count)]
+
+    def loss(p, inp):
+        total = None
+        for layer in p.w:
+            s = O.sum_(O.mul(layer.fwd(inp['x']), inp['t']))
+            total = s if total is None else O.add(total, s)
+        return total
+    return build_training_ir(Layers(), loss, {'x': [rows, d_in], 't': [rows, d_out]}, {'kind': 'sgd', 'lr': 1.0})
+
+
+def test_groups_keep_their_sums_within_the_f32_error():
+    """Twelve [256, K] x [K, 64] weight gradients in one unsplit launch sum a quarter of K each: up to K = 8192 their error
+    stays below that of the f32 split launches, over K = 12000 it would not and they stay apart (by time alone they would
+    still be grouped)."""
+    for rows, grouped in ((4096, True), (8192, True), (12000, False)):
+        nodes = backend.plan(_weight_gradients(rows, 12, 256, 64).wire_json())['nodes']
+        assert ('group of 12 GEMMs' in [n['shape'] for n in nodes]) == grouped, rows
 
 
 @pytest.mark.parametrize('n', [1, 3, 10])

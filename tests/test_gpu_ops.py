@@ -16,7 +16,9 @@ from tensorgrad_amd import backend
 from tensorgrad_amd import ir as IR
 from tensorgrad_amd import nn
 from tensorgrad_amd import ops as O
+from tensorgrad_amd.build_ir import build_training_ir
 from tensorgrad_amd.grad import append_grad
+from tensorgrad_amd.module import Module
 from tensorgrad_amd.trace import param_input, tensor_input, trace_fn
 
 pytestmark = pytest.mark.gpu
@@ -786,6 +788,43 @@ def test_matmul_long_sums_of_one_sign(M, N, K):
     a, b = _rand([M, K], 152, 0, 1), _rand([K, N], 153, 0, 1)
     got, want = run_both(_product(M, N, K, False, False), {'a': a, 'b': b})
     gemm_close(got, want, 2.0 ** -24)
+
+
+def _weight_gradients(rows, count, d_in, d_out, ins):
+    """The gradients [d_in, rows] x [rows, d_out] of `count` layers (layer i against target i % 3), as one SGD step of rate
+    1 from zero weights leaves them, and the step's lowered products."""
+    class Layers(Module):
+        def __init__(self):
+            self.w = [nn.Linear(d_in, d_out, bias=False) for _ in range(count)]
+
+    def loss(p, inp):
+        total = None
+        for i, layer in enumerate(p.w):
+            s = O.sum_(O.mul(layer.fwd(inp['x']), inp['t%d' % (i % 3)]))
+            total = s if total is None else O.add(total, s)
+        return total
+    ir = build_training_ir(Layers(), loss, {k: list(v.shape) for k, v in ins.items()}, {'kind': 'sgd', 'lr': 1.0})
+    rt = backend.NativeRuntime(ir.wire_json())
+    rt.upload_params({n: np.zeros(rt.param_numel[n], np.float32) for n in rt.param_names})
+    rt.step(ins)
+    got = {int(n.split('.')[1]): -w.reshape(d_in, d_out) for n, w in rt.download_params().items()}
+    shapes = [n['shape'] for n in rt.describe()['nodes'] if n['kind'] == 'gemm']
+    rt.destroy()
+    return got, shapes
+
+
+@pytest.mark.parametrize('rows,count,d_in,d_out', [(8192, 12, 256, 64), (4100, 12, 129, 200), (47, 12, 65, 260),
+                                                   (1003, 12, 100, 129), (33, 8, 64, 300), (130, 9, 129, 191)])
+def test_grouped_weight_gradients_split_tile(rows, count, d_in, d_out):
+    """Weight gradients in one grouped launch, over long K and at ragged rows and columns (tiles that start before their
+    own first row, a first k stage that overlaps the second), against 64 bits. Tolerance: a running sum of k values has
+    variance at most (0.5 + 1.2e-3 k) 1e-14; these launches sum at most a quarter of 8192 at once (1.72e-7)."""
+    ins = {'x': _rand([rows, d_in], 154), **{f't{q}': _rand([rows, d_out], 155 + q) for q in range(3)}}
+    got, shapes = _weight_gradients(rows, count, d_in, d_out, ins)
+    assert f'group of {count} GEMMs' in shapes
+    for i in range(count):
+        want = ins['x'].astype(np.float64).T @ ins[f't{i % 3}'].astype(np.float64)
+        gemm_close(got[i], want, 1.8e-7)
 
 
 def test_matmul_split_tile_batched_and_summed():
