@@ -885,6 +885,22 @@ bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, Gemm
 // Segments of whole 16-k stages run on the split-bf16 tile, unsplit.
 static bool sum_x3(const GemmDesc& all, int64_t seg) { return seg % kXK == 0 && x3_ok(all); }
 
+// Whether a sum runs as one unsplit launch over all of its terms' k: always below 1024 k (a launch or two less, at most
+// 10 us longer), from there where that is estimated no longer than the products apart (grouped in one launch, or split over
+// K) with an addition that reads them and writes the sum at 4 TB/s. Steps in us, in one launch and apart: 2 x [8000, 1024] x
+// [1024, 384] 99 and 115, 3 x [1600, 512] x [512, 512] 39 and 42; but 3 x [108, 384] x [384, 384] 32 and 21, 2 x [512, 1024]
+// x [1024, 512] 45 and 37, 2 x [4096, 2048] x [2048, 512] 128 and 111, 2 x [128, 8192] x [8192, 256] 239 and 33. A sum that
+// would be longer than its error allows (x3_group_tiling) stays apart.
+static bool sum_x3_pays(const GemmDesc& all, const GemmDesc* ds, int n) {
+  if (all.K < kShortK) return true;
+  constexpr double kGap = 2.0;   // us from one launch of a captured step to the next
+  double sum_us = 0.0, apart = 0.0;
+  x3_group_tiling(&all, 1, &sum_us);
+  if (gemm_group_kind(ds[0]) >= 4 && gemm_prefers_group(ds[0])) x3_group_tiling(ds, n, &apart);
+  else apart = n * x3_plan(ds[0]).us + (n - 1) * kGap;
+  return sum_us < 1e30 && sum_us <= apart + kGap + (n + 1) * 4.0 * (double)(all.M * all.N) / 4e6;
+}
+
 bool gemm_sum_ok(const GemmDesc* ds, int n) {
   if (n < 2 || n > kMaxSeg) return false;
   const GemmDesc& d0 = ds[0];
@@ -897,9 +913,10 @@ bool gemm_sum_ok(const GemmDesc* ds, int n) {
   }
   GemmDesc all = d0;
   all.K = d0.K * n;
-  if (sum_x3(all, d0.K)) return true;
+  if (sum_x3(all, d0.K)) return sum_x3_pays(all, ds, n);
   const Plan p = plan_for(all);
-  if (p.splits != 1 || p.bk != 32 && p.bk != 64 || d0.K % p.bk != 0) return false;
+  if (p.splits != 1) return false;
+  if (p.bk != 32 && p.bk != 64 || d0.K % p.bk != 0) return false;
   if (p.bm != 64 || p.bn != 64) return false;
   const bool ak = d0.sAk == 1;
   const bool bk = d0.sBk == 1 && d0.sBn != 1;

@@ -346,6 +346,42 @@ def test_groups_keep_their_sums_within_the_f32_error():
         assert ('group of 12 GEMMs' in [n['shape'] for n in nodes]) == grouped, rows
 
 
+@pytest.mark.parametrize('rows,dim,hidden,summed', [(128, 256, 8192, False), (64, 64, 65536, False), (1024, 256, 1024, False),
+                                                    (108, 512, 640, False), (4096, 256, 256, True), (8000, 384, 1024, True)])
+def test_sums_of_few_tiles_and_long_k_stay_apart(rows, dim, hidden, summed):
+    """The input gradient of a gated layer is a sum of two products over `hidden`. Few tiles over long K do better as
+    products of their own, grouped or split over K, and an addition; tiles that fill the chip are summed in one launch."""
+    class Gated(Module):
+        def __init__(self):
+            self.gate, self.up = nn.Linear(dim, hidden), nn.Linear(dim, hidden)
+            self.ln = nn.LayerNorm(dim)
+
+    def loss(p, inp):
+        x = p.ln.fwd(inp['x'])
+        return O.mean(O.square(O.mul(O.sigmoid(p.gate.fwd(x)), p.up.fwd(x))))
+    ir = build_training_ir(Gated(), loss, {'x': [rows, dim]}, {'kind': 'sgd', 'lr': 1e-3})
+    nodes = backend.plan(ir.wire_json())['nodes']
+    assert ('gemm_sum' in [n.get('ops') for n in nodes]) == summed
+
+
+def test_a_refused_sum_leaves_all_its_products_apart():
+    """The input gradient of three projections of width 384 over 108 rows: three products of their own in one grouped
+    launch, not a sum of two and one apart."""
+    class Projections(Module):
+        def __init__(self):
+            self.ln = nn.LayerNorm(384)
+            self.w = [nn.Linear(384, 384) for _ in range(3)]
+
+    def loss(p, inp):
+        x = p.ln.fwd(inp['x'])
+        a, b, c = (w.fwd(x) for w in p.w)
+        return O.mean(O.square(O.mul(O.mul(a, b), c)))
+    ir = build_training_ir(Projections(), loss, {'x': [108, 384]}, {'kind': 'sgd', 'lr': 1e-3})
+    nodes = backend.plan(ir.wire_json())['nodes']
+    assert 'gemm_sum' not in [n.get('ops') for n in nodes]
+    assert sum(n['shape'] == 'group of 3 GEMMs' for n in nodes) == 3   # forward, input gradient, weight gradients
+
+
 @pytest.mark.parametrize('n', [1, 3, 10])
 def test_forward_of_one_row_lowers_with_epilogues(n):
     """C1's forward at batch n (compileForward's shapes): every product is tiny and takes
