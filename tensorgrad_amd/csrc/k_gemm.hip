@@ -1431,20 +1431,26 @@ __global__ void k_segment_finish(const double* __restrict__ part, int64_t N, int
 // Small vocabularies (V * rows <= kScatterScanMax), and larger ones over few rows, need no
 // sort: block (v, column chunk) of four wavefronts runs scatter_scan_block (scatter_dev.h).
 // One launch, no workspace. With few rows the sort's one block and its three launches cost
-// more than every token's block reading all the row ids (from L2).
+// more than every block reading all the row ids (from L2): 5003 tokens, 2048 rows of 256 47 us
+// sorted, 18 scanned; 8192 of either 157 and 48. A block costs about 1.9 ns of the chip's time and 0.45 ps
+// a row whatever it adds up, so where one column a thread would make more than 8192 blocks a thread takes up to
+// kScatterWideCols (7000 tokens of 1300: 700 rows 41 us sorted, 86 one column a thread, 43 so; 1500 rows 61, 100, 56; 8192
+// tokens of 1024: 1024 rows 47, 70, 40; 8192 rows 191, 174, 119).
 constexpr int64_t kScatterScanMax = int64_t(1) << 22;
-constexpr int64_t kScatterFewRows = 8192, kScatterScanFew = int64_t(1) << 26;
+constexpr int64_t kScatterFewRows = 8192;
+constexpr int kScatterWideCols = 8;
 
+template <int C>
 __global__ __launch_bounds__(256) void k_scatter_scan(const int32_t* __restrict__ idx, int64_t rows,
                                                       const float* __restrict__ dy, int64_t N,
                                                       float* __restrict__ out) {
   __shared__ ScatterScanLds<4> L;
-  scatter_scan_block<4>(idx, rows, dy, N, out, (int)blockIdx.x, blockIdx.y * 256ll, L);
+  scatter_scan_block<4, C>(idx, rows, dy, N, out, (int)blockIdx.x, blockIdx.y * (256ll * C), L);
 }
 
-inline bool scatter_scans(int64_t rows, int64_t V) {
-  return V * rows <= (rows <= kScatterFewRows ? kScatterScanFew : kScatterScanMax);
-}
+inline bool scatter_scans(int64_t rows, int64_t V) { return V * rows <= kScatterScanMax || rows <= kScatterFewRows; }
+
+inline bool scatter_scans_wide(int64_t V, int64_t N) { return N > 256 && V * ((N + 255) / 256) > 8192; }
 
 inline int grid_for(int64_t n) {
   int64_t b = (n + 255) / 256;
@@ -1465,7 +1471,7 @@ void gather_rows(const int32_t* idx, int64_t rows, const float* table, int64_t V
   klaunch(k_gather_rows, grid_for(rows * N), 256, 0, st, idx, rows, table, V, N, out);
 }
 
-bool scatter_scan_form(int64_t rows, int64_t V) { return scatter_scans(rows, V); }
+bool scatter_scan_form(int64_t rows, int64_t V, int64_t N) { return scatter_scans(rows, V) && !scatter_scans_wide(V, N); }
 
 int64_t scatter_workspace_bytes(int64_t rows, int64_t V, int64_t N) {
   if (scatter_scans(rows, V)) return 0;
@@ -1479,9 +1485,12 @@ void scatter_rows(const int32_t* idx, int64_t rows, const float* dy, int64_t V, 
   if (V * N <= 0) return;
   if (V > kMaxBucketV || rows >= (int64_t(1) << 31)) throw std::runtime_error("scatter_rows: V or rows too large");
   if (scatter_scans(rows, V)) {
-    const int64_t ny = (N + 255) / 256;
+    const bool wide = scatter_scans_wide(V, N);
+    const int64_t cols = wide ? 256 * kScatterWideCols : 256, ny = (N + cols - 1) / cols;
     if (ny > 65535) throw std::runtime_error("scatter_rows: N too large");
-    klaunch(k_scatter_scan, dim3((unsigned)V, (unsigned)ny), 256, 0, st, idx, rows, dy, N, out);
+    const dim3 grid((unsigned)V, (unsigned)ny);
+    if (wide) klaunch(k_scatter_scan<kScatterWideCols>, grid, 256, 0, st, idx, rows, dy, N, out);
+    else klaunch(k_scatter_scan<1>, grid, 256, 0, st, idx, rows, dy, N, out);
     return;
   }
   const int64_t items = (rows + kSeg - 1) / kSeg + V;

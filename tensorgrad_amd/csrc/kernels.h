@@ -364,9 +364,9 @@ void gather_rows(const int32_t* idx, int64_t rows, const float* table, int64_t V
 // order, f64 accumulation (V <= 8192); `work` must hold scatter_workspace_bytes(...)
 // bytes, 256-byte aligned.
 int64_t scatter_workspace_bytes(int64_t rows, int64_t V, int64_t N);
-// The sort-free form (small V * rows): one launch, no workspace; the form a column-sum
-// launch can run beside its sums (ColSumScatter).
-bool scatter_scan_form(int64_t rows, int64_t V);
+// The sort-free form with a column a thread (small V * rows, or few rows of a table that is not
+// wide): one launch, no workspace; the form a column-sum launch can run beside its sums (ColSumScatter).
+bool scatter_scan_form(int64_t rows, int64_t V, int64_t N);
 void scatter_rows(const int32_t* idx, int64_t rows, const float* dy, int64_t V, int64_t N, float* out, void* work,
                   hipStream_t st);
 

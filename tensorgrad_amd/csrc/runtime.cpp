@@ -4034,7 +4034,7 @@ void Runtime::lower_op(int i) {
       if (va.dims.size() == 2 && va.dims[0] == V && va.dims[1] == rows && va.strides[0] == 1 && va.strides[1] == V &&
           view_[b].contiguous() && V <= 8192) {
         const DeferredScatter sc{i, fld(asrc, "indices"), b, out, rows, V, N, n.shape};
-        if (use_gemm_group_ && use_colsum_scatter_ && deferred_scatter_.empty() && tgk::scatter_scan_form(rows, V) &&
+        if (use_gemm_group_ && use_colsum_scatter_ && deferred_scatter_.empty() && tgk::scatter_scan_form(rows, V, N) &&
             only_optimizer_reads(out)) {
           deferred_scatter_.push_back(sc);
           return;

@@ -64,6 +64,24 @@ def test_embedding_gradient_joins_the_column_sums(monkeypatch):
     assert not any('+ scatter' in n['shape'] for n in nodes)
 
 
+@pytest.mark.parametrize('V,rows,N,joins', [(5003, 2048, 256, True), (8192, 8192, 256, True), (4096, 2048, 512, True),
+                                            (8192, 1300, 257, False), (7000, 700, 1300, False), (4097, 2048, 512, False)])
+def test_wide_embedding_gradients_over_few_rows(V, rows, N, joins):
+    """The scanning form of an embedding gradient joins the column sums' launch, a block per token and 256 columns that reads
+    every row id. For wide tables those blocks would take longer than the sort, so they run a launch of their own with
+    several columns a thread, still without a workspace."""
+    class Embed(Module):
+        def __init__(self):
+            self.emb, self.ln = nn.Embedding(V, N), nn.LayerNorm(N)
+
+    def loss(p, inp):
+        return O.mean(O.square(p.ln.fwd(p.emb.fwd(inp['t']))))
+    ir = build_training_ir(Embed(), loss, {'t': {'shape': [rows], 'dtype': 'i32'}}, {'kind': 'sgd', 'lr': 1e-3})
+    nodes = backend.plan(ir.wire_json())['nodes']
+    assert any('+ scatter' in n['shape'] for n in nodes) == joins
+    assert ('scatter' in [n['kind'] for n in nodes]) != joins
+
+
 @pytest.mark.parametrize('key', ['mlp_sin', 'char_mlp', 'cnn', 'transformer'])
 def test_loss_mean_joins_the_column_sums(monkeypatch, key):
     """The loss mean (a row group reducing the per-sample losses to the output scalar) runs

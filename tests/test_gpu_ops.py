@@ -914,6 +914,9 @@ def test_matmul_batched_head_views():
     (2, 8, 64, False),
     (8000, 40, 8192, False),   # few rows: every token's block scans them all
     (2000, 24, 8193, False),   # one row more: sorted
+    (8192, 257, 1024, False),  # several columns a thread: one past a block's width, a part of a chunk
+    (1000, 2300, 5000, False), # two blocks of eight columns a thread, the second with a part of one
+    (4097, 512, 1100, True),   # and one token owning most rows
 ])
 def test_embedding_gather_and_scatter(V, N, rows, skew):
     rng = np.random.default_rng(18)
