@@ -221,38 +221,41 @@ __device__ __forceinline__ void tile_finish(const GemmArgs& g, const Epi& epi, f
       return;
     }
     if constexpr (Epi::kPrefetch) {
-      // An epilogue that reads other tensors: every one of its loads for the wave's
-      // accumulator values is issued first (clamped to an element in range), then the values
-      // are computed and stored. Interleaved, each load would wait for the stores before it
-      // (the outputs may alias the inputs as far as the compiler knows): one memory latency
-      // per value.
-      typename Epi::Pre pre[TM][TN][16];
+      // An epilogue that reads other tensors: the loads of a 32 x 32 tile's values (clamped to an element in range) are
+      // issued together, those of the next tile before this one's values are computed and stored. Interleaved, each load
+      // would wait for the stores before it (the outputs may alias the inputs as far as the compiler knows): one memory
+      // latency per value. All tiles' at once do not fit the registers of a wavefront with four tiles: six operations
+      // and column sums after [65536, 319] x [319, 256] spilled 87 registers, 203 us, so 98; five after [4096, 512] x
+      // [512, 2048] 96 and 60.
+      typename Epi::Pre pre[2][16];
+      auto fetch = [&](int t) {
+        const int i = t / TN, j = t % TN;
+        const int64_t gn = EDGE ? min((int64_t)(nw + j * 32 + lrow), d.N - 1) : nw + j * 32 + lrow;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int r = 0; r < 16; ++r) pre[t & 1][r] = epi.load(d, EDGE ? min(row(i, r), d.M - 1) : row(i, r), gn);
+      };
+      // kColSum: the epilogue also returns the value of an output whose column sums are wanted: each
+      // lane totals its column over the wave's rows it holds (f64, in (i, r) order), the two
+      // lane halves (h = 0, 1: the other rows of the same column) are added, and lanes of
+      // h = 0 store the wave's partial row (one batch: z = 0).
+      double cs[TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t gn = EDGE ? min((int64_t)(nw + j * 32 + lrow), d.N - 1) : nw + j * 32 + lrow;
+      for (int j = 0; j < TN; ++j) cs[j] = 0.0;
+      fetch(0);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) pre[i][j][r] = epi.load(d, EDGE ? min(row(i, r), d.M - 1) : row(i, r), gn);
+      for (int t = 0; t < TM * TN; ++t) {
+        if (t + 1 < TM * TN) fetch(t + 1);
+        const int i = t / TN, j = t % TN;
+        const int64_t gn = nw + j * 32 + lrow;
+        if (!col_ok(gn)) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          if (!row_ok(row(i, r))) continue;
+          const float v = epi(d, z0, z1, row(i, r), gn, acc[i][j][r], pre[t & 1][r]);
+          if (Epi::kColSum) cs[j] += (double)v;
         }
+      }
       if constexpr (Epi::kColSum) {
-        // The epilogue also returns the value of an output whose column sums are wanted: each
-        // lane totals its column over the wave's rows it holds (f64, in (i, r) order), the two
-        // lane halves (h = 0, 1: the other rows of the same column) are added, and lanes of
-        // h = 0 store the wave's partial row (one batch: z = 0).
-        double cs[TN];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) cs[j] = 0.0;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const int64_t gn = nw + j * 32 + lrow;
-            if (!col_ok(gn)) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (row_ok(row(i, r))) cs[j] += (double)epi(d, z0, z1, row(i, r), gn, acc[i][j][r], pre[i][j][r]);
-          }
         const int64_t prow = (int64_t)tm * WGM + wrow;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
@@ -260,18 +263,7 @@ __device__ __forceinline__ void tile_finish(const GemmArgs& g, const Epi& epi, f
           const int64_t gn = nw + j * 32 + lrow;
           if (h == 0 && col_ok(gn)) g.colsum[prow * d.N + gn] = t;
         }
-        return;
       }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t gn = nw + j * 32 + lrow;
-          if (!col_ok(gn)) continue;
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (row_ok(row(i, r))) epi(d, z0, z1, row(i, r), gn, acc[i][j][r], pre[i][j][r]);
-        }
     } else {
       float* C = d.C + z0 * d.sCz0 + z1 * d.sCz1;
 #pragma unroll

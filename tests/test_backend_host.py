@@ -12,6 +12,7 @@ from tensorgrad_amd import ops as O
 from tensorgrad_amd.build_ir import build_forward_ir, build_training_ir
 from tensorgrad_amd.module import Module
 
+HERE = os.path.dirname(os.path.abspath(__file__))
 HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), 'include', 'tg.h')
 
 
@@ -398,6 +399,55 @@ def test_a_refused_sum_leaves_all_its_products_apart():
     nodes = backend.plan(ir.wire_json())['nodes']
     assert 'gemm_sum' not in [n.get('ops') for n in nodes]
     assert sum(n['shape'] == 'group of 3 GEMMs' for n in nodes) == 3   # forward, input gradient, weight gradients
+
+
+def test_epilogues_fit_the_registers(tmp_path):
+    """Generated kernels of products on 128 x 128 split-bf16 tiles whose epilogues load several operands and add up
+    columns (a loss's gradient after a concatenation's product, a gated layer's after a plain one) spill no registers."""
+    import subprocess
+    import sys
+    source = tmp_path / 'kernels.hip'
+    code = '''
+from tensorgrad_amd import backend, nn, ops as O
+from tensorgrad_amd.build_ir import build_training_ir
+from tensorgrad_amd.module import Module
+
+class Skip(Module):
+    def __init__(self):
+        self.a, self.b = nn.Linear(63, 256), nn.Linear(319, 256)
+
+def skip(p, inp):
+    x = inp['x']
+    return O.mean(O.square(O.sub(p.b.fwd(O.concat([O.relu(p.a.fwd(x)), x], 1)), inp['t'])))
+
+class Gated(Module):
+    def __init__(self):
+        self.gate, self.up, self.down = nn.Linear(512, 2048), nn.Linear(512, 2048), nn.Linear(2048, 512)
+
+def gated(p, inp):
+    x = inp['x']
+    return O.mean(O.square(O.sub(p.down.fwd(O.mul(O.sigmoid(p.gate.fwd(x)), p.up.fwd(x))), inp['t'])))
+
+for model, loss, ins in ((Skip(), skip, {'x': [65536, 63], 't': [65536, 256]}),
+                         (Gated(), gated, {'x': [4096, 512], 't': [4096, 512]})):
+    ir = build_training_ir(model, loss, ins, {'kind': 'sgd', 'lr': 1e-3})
+    ops = [n.get('ops', '') for n in backend.plan(ir.wire_json())['nodes']]
+    assert any('gemm' in o and o.endswith(',colsum') and o.count(',') >= 5 for o in ops), ops
+'''
+    root = os.path.dirname(HERE)
+    subprocess.run([sys.executable, '-c', code], check=True, cwd=root, env=dict(os.environ, TG_JIT_DUMP=str(source)))
+    out = subprocess.run(['/opt/rocm/bin/hipcc', '--offload-arch=gfx950', '-O3', '-std=c++17', '-ffp-contract=off', '-Xclang',
+                          '-target-feature', '-Xclang', '-packed-fp32-ops', '--cuda-device-only', '-c', str(source), '-o',
+                          os.devnull, '-Rpass-analysis=kernel-resource-usage'], capture_output=True, text=True,
+                         check=True).stderr
+    name, seen = '', 0
+    for line in out.splitlines():
+        if m := re.search(r'Function Name: (\w+)', line):
+            name = m.group(1)
+        elif (m := re.search(r'VGPRs Spill: (\d+)', line)) and name.startswith('tg_g'):
+            seen += 1
+            assert m.group(1) == '0', f'{name} spills {m.group(1)} registers'
+    assert seen >= 4
 
 
 @pytest.mark.parametrize('n', [1, 3, 10])
