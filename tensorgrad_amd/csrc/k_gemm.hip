@@ -810,6 +810,27 @@ void gemm(const GemmDesc& d, float* work, hipStream_t st) {
   if (p.splits > 1) add_splits(p.splits);
 }
 
+static std::string x3_tile_name(const XTiling& t, int splits) {
+  return "x3 " + std::to_string(t.bm) + "x" + std::to_string(t.bn) + "/" + std::to_string(t.kg) +
+         (splits > 1 ? " split " + std::to_string(splits) : std::string());
+}
+
+std::string gemm_tile(const GemmDesc& d) {
+  SkinnyPlan sk;
+  if (gemm_is_tiny(d)) return "tiny";
+  if (gemm_is_smallk(d)) return "smallk";
+  if (skinny_plan(d, sk)) return "skinny";
+  if (x3_ok(d)) {
+    const XPlan xp = x3_plan(d);
+    return x3_tile_name(kXTilings[xp.tiling], xp.splits);
+  }
+  return "f32";
+}
+
+std::string gemm_group_tile(const GemmDesc* ds, int n, int kind) {
+  return kind >= 4 ? x3_tile_name(kXTilings[x3_group_tiling(ds, n, nullptr)], 1) : "f32";
+}
+
 // ---- products over a concatenation along k ---------------------------------------------
 // A = [A0 | A1] along k: k < k0 from d.A (row stride d.sAm, 16-byte aligned rows), the rest
 // from c.a1 (row stride c.lda1, any alignment). One launch of 128 x 128 tiles whose stages
@@ -876,6 +897,8 @@ bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, Gemm
   return true;
 }
 
+std::string gemm_cat_tile(const GemmDesc& d, const GemmCat& c) { return cat_x3(d, c) ? "x3 128x128/1" : "f32"; }
+
 // ---- sums of products ------------------------------------------------------------------
 // C = sum_s A_s B_s in one launch: the products' k ranges are stages of one GEMM whose
 // stage st reads segment st / (K_s / BK) through its own bases. Every segment shares the
@@ -923,6 +946,12 @@ bool gemm_sum_ok(const GemmDesc* ds, int n) {
   for (int s = 0; s < n; ++s)
     if (!dma_ok(ds[s], Plan{p.bm, p.bn, p.bk, 1, ds[s].K}, ak, bk)) return false;
   return true;
+}
+
+std::string gemm_sum_tile(const GemmDesc* ds, int n) {
+  GemmDesc all = ds[0];
+  all.K = ds[0].K * n;
+  return sum_x3(all, ds[0].K) ? x3_tile_name(kXTilings[x3_group_tiling(&all, 1, nullptr)], 1) : "f32";
 }
 
 void gemm_sum(const GemmDesc* ds, int n, hipStream_t st) {

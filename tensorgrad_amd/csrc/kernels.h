@@ -347,6 +347,12 @@ struct GemmCat {
 bool gemm_cat_ok(const GemmDesc& d, const GemmCat& c);
 void gemm_cat(const GemmDesc& d, const GemmCat& c, hipStream_t st);
 bool gemm_cat_epi_cfg(const GemmDesc& d, const GemmCat& c, GemmEpiCfg& cfg, gd::GemmArgs& g, int64_t& blocks);
+// The kernels these launch, for descriptions: "x3 ROWSxCOLUMNS/GROUPS[ split SPLITS]" on the split-bf16 tile, "f32" on f32
+// tiles, or "tiny", "smallk", "skinny".
+std::string gemm_tile(const GemmDesc& d);
+std::string gemm_cat_tile(const GemmDesc& d, const GemmCat& c);
+std::string gemm_sum_tile(const GemmDesc* ds, int n);
+std::string gemm_group_tile(const GemmDesc* ds, int n, int kind);
 // True when d on its own would run one pass of tiles that does not fill the chip twice; the
 // grouped launch's tiling (on f32 tiles: its k-stage depth) follows its own tile count.
 bool gemm_prefers_group(const GemmDesc& d);

@@ -194,6 +194,7 @@ struct Node {
   double flops = 0, bytes = 0;      // algorithmic work per launch
   std::string shape;
   std::string detail;  // fused groups: member op kinds in program order
+  std::string tile;    // products: the kernel that runs them
   bool ws = false;     // bind() reads cur_ws_ / cur_counters_ (rebound for the scratch-only step)
   bool partials = false;   // reads column partials another launch of the step writes (in no tensor of `reads`)
   std::function<void(hipStream_t)> launch;   // bound after allocation
@@ -3237,6 +3238,7 @@ void Runtime::lower_gemm_epi(int op, const tgk::GemmDesc& d, int a, int b, int o
   for (int t : gp.outs) n.writes.push_back(root(t));
   if (store_c) n.writes.push_back(root(out));
   n.flops = 2.0 * (double)d.M * d.N * d.K * d.batch;
+  n.tile = is_cat ? tgk::gemm_cat_tile(d, tgk::GemmCat{nullptr, cf.k0, cf.k1}) : tgk::gemm_tile(d);
   n.bytes = 4.0 * ((double)T_[a].numel + T_[b].numel) + (store_c ? 4.0 * T_[out].numel : 0.0);
   for (auto& e : gp.ext) if (root(e.first) != out) n.bytes += 4.0 * T_[e.first].numel;
   for (int t : gp.outs) n.bytes += 4.0 * T_[t].numel;
@@ -3493,6 +3495,7 @@ void Runtime::lower_gemm_sum(int add_op) {
   n.writes.push_back(root(out));
   n.flops = fl;
   n.bytes = by;
+  n.tile = tgk::gemm_sum_tile(ds.data(), (int)ds.size());
   n.shape = shape_str(T_[out].shape) + " sum of " + std::to_string(terms.size()) + " products";
   n.bind = [this, ds, as, bs, out]() -> std::function<void(hipStream_t)> {
     std::vector<tgk::GemmDesc> dd = ds;
@@ -3527,6 +3530,9 @@ void Runtime::emit_gemm_group(const std::vector<DeferredGemm>& grp) {
   n.flops = fl;
   n.bytes = by;
   n.shape = "group of " + std::to_string(grp.size()) + " GEMMs";
+  std::vector<tgk::GemmDesc> gds;
+  for (const DeferredGemm& g : grp) gds.push_back(g.d);
+  n.tile = tgk::gemm_group_tile(gds.data(), (int)gds.size(), kind);
   n.bind = [this, grp, kind]() -> std::function<void(hipStream_t)> {
     std::vector<tgk::GemmDesc> ds;
     for (const DeferredGemm& g : grp) {
@@ -4065,6 +4071,7 @@ void Runtime::lower_op(int i) {
       }
       rd(cf.src0); rd(cf.src1); rd(b);
       n.detail = "gemm_cat";
+      n.tile = tgk::gemm_cat_tile(d, tgk::GemmCat{nullptr, cf.k0, cf.k1});
       n.bytes = 4.0 * (T_[a].numel + T_[b].numel + to.numel);
       n.bind = [=]() -> std::function<void(hipStream_t)> {
         check_cat_spans(d, cf, b, out, true);
@@ -4091,6 +4098,7 @@ void Runtime::lower_op(int i) {
         g.sAk = g.M;
         ws = std::max(ws, tgk::gemm_workspace_floats(g));
         ds.push_back(g);
+        n.tile += (s ? ", " : "") + tgk::gemm_tile(g);
         rd(cat_src[s]);
       }
       rd(b);
@@ -4151,6 +4159,7 @@ void Runtime::lower_op(int i) {
       }
     }
     workspace_bytes_ = std::max(workspace_bytes_, (size_t)ws * 4);
+    n.tile = tgk::gemm_tile(d);
     n.bytes = 4.0 * (T_[a].numel + T_[b].numel + to.numel);
     n.ws = ws > 0;
     n.bind = [=]() -> std::function<void(hipStream_t)> {
@@ -4824,6 +4833,7 @@ std::string Runtime::describe() {
       << (n.op >= 0 ? kinds_[n.op] : "") << "\",\"shape\":\"" << n.shape << "\",\"flops\":" << n.flops
       << ",\"bytes\":" << n.bytes;
     if (!n.detail.empty()) o << ",\"ops\":\"" << n.detail << "\"";
+    if (!n.tile.empty()) o << ",\"tile\":\"" << n.tile << "\"";
     o << "}";
   }
   o << "],\"arena_bytes\":" << arena_bytes_ << ",\"workspace_bytes\":" << workspace_bytes_

@@ -6,7 +6,8 @@ import numpy as np
 import pytest
 
 import pyoracle
-from tensorgrad_amd import configs, nn
+from _helpers import HipBuffers
+from tensorgrad_amd import backend, configs, nn
 from tensorgrad_amd import ops as O
 from tensorgrad_amd.backend import BackendError
 from tensorgrad_amd.build_ir import build_training_ir
@@ -39,6 +40,50 @@ def test_step_matches_oracle_and_returns_completed():
         _close(r.loss, o.step(b))
     assert t.param_names == ['l1.W', 'l1.b', 'l2.W', 'l2.b', 'l3.W', 'l3.b']
     t.destroy()
+
+
+def _sin(n):
+    inputs = {'x': [n, 1], 'y': [n, 1]}
+    r = np.random.default_rng(n)
+    batches = [{k: r.uniform(-1, 1, (n, 1)).astype(np.float32) for k in 'xy'} for _ in range(4)]
+    return build_training_ir(configs.SinMLP(16), configs.sin_mlp_loss, inputs, {'kind': 'adam', 'lr': 1e-3}), batches
+
+
+def _dropout_transformer(_):
+    cfg = configs.small_variant('transformer')
+    return build_training_ir(cfg.make_model(), cfg.loss, cfg.inputs, cfg.optimizer), configs.batches(cfg, 4)
+
+
+@pytest.mark.parametrize('make,n', [(_sin, 257), (_sin, 131072), (_sin, 131073), (_dropout_transformer, 0)])
+def test_steps_fed_from_host_slots_and_device_interleave(make, n):
+    """Batches from host arrays (fetched by the captured step, or copied ahead of it above 1 MiB: 131072 and 131073 points
+    are just that and one more), from staged slots and from device pointers, in any order on one runtime: the same losses
+    and weights, bit for bit, as the same batches all from host arrays, so no step sees another's batch, seed or rate."""
+    ir, batches = make(n)
+    ref, mixed = backend.NativeRuntime(ir.wire_json()), backend.NativeRuntime(ir.wire_json())
+    p0 = ir.initial_params(7)
+    for rt in (ref, mixed):
+        rt.upload_params(p0)
+    for slot in (0, 1):
+        mixed.stage_batch(slot, batches[slot])
+    held = [HipBuffers(b) for b in batches[:2]]
+    ways = ['host', 'slot', 'host', 'device', 'slot', 'device', 'host', 'host', 'slot', 'slot', 'device', 'host']
+    for i, way in enumerate(ways):
+        q = i % 2 if way != 'host' else i % 4
+        want = ref.step(batches[q])
+        if way == 'host':
+            got = mixed.step(batches[q])
+        elif way == 'slot':
+            got = mixed.step_staged(q)
+        else:
+            got = mixed.step_device(held[q].names, held[q].ptrs, held[q].nbytes)
+        assert np.float32(got).view(np.uint32) == np.float32(want).view(np.uint32), (i, way, got, want)
+    a, b = ref.download_params(), mixed.download_params()
+    assert all(np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)) for k in a)
+    for h in held:
+        h.free()
+    ref.destroy()
+    mixed.destroy()
 
 
 def test_upload_download_roundtrip_and_strictness():

@@ -689,7 +689,12 @@ def test_matmul(case):
 # stage more or less, every tiling (few tiles by four groups, 128-wide ones), split K, a batch with strided views
 X3 = [(64, 64, 32), (65, 64, 33), (127, 129, 47), (128, 128, 48), (129, 191, 63), (191, 127, 65), (64, 300, 95),
       (1000, 64, 257), (300, 5003, 64), (128, 64, 1024), (130, 70, 1100), (256, 256, 9000), (4100, 260, 81),
-      (2048, 2050, 130)]
+      (2048, 2050, 130), (65, 257, 33), (127, 300, 47), (191, 260, 65), (130, 140, 1100)]
+
+
+def _tiles(body):
+    """The kernels that a body's products are planned on."""
+    return [n['tile'] for n in backend.plan(IR.dumps(wire(trace_fn(body))))['nodes'] if 'tile' in n]
 
 
 def _product(M, N, K, ta, tb):
@@ -708,6 +713,9 @@ def test_matmul_split_tile(M, N, K, ta, tb):
     a, b = _rand([K, M] if ta else [M, K], 141), _rand([N, K] if tb else [K, N], 142)
     got, want = run_both(_product(M, N, K, ta, tb), {'a': a, 'b': b})
     gemm_close(got, want, 2.0 ** -24 * (4 + (K / 16) ** 0.5))
+    # few columns that fill no tile, or a short odd k, run on the skinny kernel where its loads are coalesced
+    skinny = not tb and (ta or K % 4 == 0) and (N <= 128 and N % 64 or K < 128 and K % 32 and N <= 256)
+    assert [t.split()[0] for t in _tiles(_product(M, N, K, ta, tb))] == ['skinny' if skinny else 'x3']
 
 
 def test_matmul_split_tile_wide_values():
@@ -725,7 +733,7 @@ def test_matmul_split_tile_wide_values():
     assert np.all(got[:, 7] == 0) and np.array_equal(got[:, 9], a[:, 5])
 
 
-@pytest.mark.parametrize('M,N,K', [(130, 70, 40), (300, 256, 300), (256, 256, 2050)])
+@pytest.mark.parametrize('M,N,K', [(130, 270, 40), (300, 256, 300), (256, 256, 2050), (130, 129, 130)])
 def test_matmul_split_tile_infinities(M, N, K):
     """Infinities, NaN and values that round to infinity in bf16 give what f32 products give, and leave the other rows
     and columns alone."""
@@ -734,6 +742,7 @@ def test_matmul_split_tile_infinities(M, N, K):
     a[20] = 0
     a[20, 1], b[1] = 3.4e38, np.float32(1e-3) * b[1]
     got, want = run_both(_product(M, N, K, False, False), {'a': a, 'b': b})
+    assert _tiles(_product(M, N, K, False, False))[0].startswith('x3')
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(got)], want[np.isinf(want)])
     ok = np.isfinite(want)
@@ -808,7 +817,7 @@ def _weight_gradients(rows, count, d_in, d_out, ins):
     rt.upload_params({n: np.zeros(rt.param_numel[n], np.float32) for n in rt.param_names})
     rt.step(ins)
     got = {int(n.split('.')[1]): -w.reshape(d_in, d_out) for n, w in rt.download_params().items()}
-    shapes = [n['shape'] for n in rt.describe()['nodes'] if n['kind'] == 'gemm']
+    shapes = [(n['shape'], n['tile'][:2]) for n in rt.describe()['nodes'] if n['kind'] == 'gemm']
     rt.destroy()
     return got, shapes
 
@@ -821,7 +830,7 @@ def test_grouped_weight_gradients_split_tile(rows, count, d_in, d_out):
     variance at most (0.5 + 1.2e-3 k) 1e-14; these launches sum at most a quarter of 8192 at once (1.72e-7)."""
     ins = {'x': _rand([rows, d_in], 154), **{f't{q}': _rand([rows, d_out], 155 + q) for q in range(3)}}
     got, shapes = _weight_gradients(rows, count, d_in, d_out, ins)
-    assert f'group of {count} GEMMs' in shapes
+    assert (f'group of {count} GEMMs', 'x3') in shapes
     for i in range(count):
         want = ins['x'].astype(np.float64).T @ ins[f't{i % 3}'].astype(np.float64)
         gemm_close(got[i], want, 1.8e-7)
@@ -837,6 +846,7 @@ def test_matmul_split_tile_batched_and_summed():
         return O.matmul(q, O.swap_axes(k, -1, -2))
     got, want = run_both(scores, {'x': x, 'y': y})
     gemm_close(got, want)
+    assert _tiles(scores)[0].startswith('x3')
 
     M, N, K = 192, 70, 48
     ins = {f'a{q}': _rand([M, K], 150 + q) for q in range(3)}
@@ -845,6 +855,8 @@ def test_matmul_split_tile_batched_and_summed():
     def total():
         ps = [O.matmul(tensor_input(f'a{q}', [M, K]), O.swap_axes(tensor_input(f'b{q}', [N, K]), -1, -2)) for q in range(3)]
         return O.relu(O.add(O.add(ps[0], ps[1]), ps[2]))
+    nodes = backend.plan(IR.dumps(wire(trace_fn(total))))['nodes']
+    assert [n['tile'][:2] for n in nodes if n.get('ops') == 'gemm_sum'] == ['x3']
     for inf in (False, True):
         if inf:
             ins['a1'][100, 20] = np.inf
@@ -854,7 +866,7 @@ def test_matmul_split_tile_batched_and_summed():
         gemm_close(got[ok], want[ok])
 
 
-@pytest.mark.parametrize('M,k0,k1,N', [(128, 32, 16, 128), (300, 64, 17, 130), (2000, 32, 63, 256), (129, 96, 32, 200)])
+@pytest.mark.parametrize('M,k0,k1,N', [(128, 32, 16, 128), (300, 64, 17, 132), (2000, 32, 63, 256), (129, 96, 32, 200)])
 def test_concat_product_split_tile(M, k0, k1, N):
     """A product over two sources with 16 or more k in the second, whole and with an infinity in each source."""
     ins = {'s0': _rand([M, k0], 171), 's1': _rand([M, k1], 172), 'w': _rand([k0 + k1, N], 173)}
@@ -862,6 +874,8 @@ def test_concat_product_split_tile(M, k0, k1, N):
     def body():
         return O.matmul(O.concat([tensor_input('s0', [M, k0]), tensor_input('s1', [M, k1])], -1),
                         tensor_input('w', [k0 + k1, N]))
+    nodes = backend.plan(IR.dumps(wire(trace_fn(body))))['nodes']
+    assert [(n['ops'], n['tile'][:2]) for n in nodes if n['kind'] == 'gemm'] == [('gemm_cat', 'x3')]
     for inf in (False, True):
         if inf:
             ins['s0'][5, 3] = ins['s1'][100, k1 - 1] = np.inf
@@ -869,6 +883,39 @@ def test_concat_product_split_tile(M, k0, k1, N):
         assert np.array_equal(np.isinf(got), np.isinf(want)) and not np.isnan(got).any()
         ok = np.isfinite(want)
         gemm_close(got[ok], want[ok])
+
+
+@pytest.mark.parametrize('M,k0,k1,N,tile', [(16001, 0, 250, 250, 'x3 128x128/2'), (16500, 0, 300, 258, 'x3 128x64/1'),
+                                            (9000, 0, 300, 150, 'x3 128x64/2'), (1003, 0, 300, 130, 'x3 64x64/2'),
+                                            (300, 96, 63, 132, 'x3 128x128/1'), (2500, 32, 16, 260, 'x3 128x128/1')])
+def test_split_tile_epilogue_with_column_sums(M, k0, k1, N, tile):
+    """A loss's gradient in the epilogue of the last product, at rows and columns that fill no tile, with the bias gradient
+    from its column partials: against 64 bits. The product reads one source, or a concatenation of two."""
+    class Last(Module):
+        def __init__(self):
+            self.l = nn.Linear(k0 + k1, N)
+
+    def loss(p, inp):
+        x = O.concat([inp['x0'], inp['x1']], 1) if k0 else inp['x1']
+        return O.mean(O.square(O.sub(p.l.fwd(x), inp['t'])))
+    ins = {'x1': _rand([M, k1], 181), 't': _rand([M, N], 182)}
+    if k0:
+        ins['x0'] = _rand([M, k0], 183)
+    ir = build_training_ir(Last(), loss, {k: list(v.shape) for k, v in ins.items()}, {'kind': 'sgd', 'lr': float(M * N)})
+    rt = backend.NativeRuntime(ir.wire_json())
+    w, b = _rand([k0 + k1, N], 184) / np.float32((k0 + k1) ** 0.5), _rand([N], 185)
+    rt.upload_params({'l.W': w, 'l.b': b})
+    got_loss = rt.step(ins)
+    nodes = [n for n in rt.describe()['nodes'] if n.get('ops', '').endswith(',colsum')]
+    assert len(nodes) == 1 and nodes[0]['tile'] == tile and (k0 == 0 or 'gemm_cat' in nodes[0]['ops'])
+    p = rt.download_params()
+    rt.destroy()
+    x = np.concatenate([ins['x0'], ins['x1']], 1) if k0 else ins['x1']
+    d = x.astype(np.float64) @ w + b - ins['t']
+    assert abs(got_loss - (d * d).mean()) <= 1e-6 * (d * d).mean()
+    # the updates are w - M N g and b - M N g: they round a few times more, by at most 2^-24 of themselves
+    for name, before, g in (('l.W', w, 2 * x.astype(np.float64).T @ d), ('l.b', b, 2 * d.sum(0))):
+        gemm_close(p[name].reshape(before.shape), before - g, 1e-6)
 
 
 @pytest.mark.parametrize('sa,sb,ta', [([256, 1], [1, 64], False), ([256, 64], [64, 1], False),
