@@ -1,7 +1,7 @@
 """Benchmark: train steps/sec (fwd + bwd + Adam) per config on one MI355X.
 
 Prints ONE JSON line. `value` is the headline config's steps/s (default: the transformer,
-C5, the config the north star's roofline targets are stated on) with every batch already
+C5) with every batch already
 resident in HBM when the timed region starts (batches are staged into device slots
 beforehand); each timed step still uploads the per-step optimizer scalars and PRNG seed,
 replays the captured step graph and reads the 4-byte loss back (the API's semantics).
@@ -11,8 +11,9 @@ per-family kernel rates. Kernel rates come from the kernels' own durations insid
 steps: every kernel of a step is dispatched with start / end events of its own
 (tg_profile_kernels), the quantity a profiler's kernel trace reports, without the gaps
 between launches. `roofline` is for the dominant kernel family of the headline config
-(its f32 MFMA GEMMs), `roofline_mfma_all` for every MFMA kernel (GEMMs and fused
-attention); `cpu_baseline` is the CPU oracle (a C++ restatement of the reference's CPU
+(its GEMMs: each launch against the peak of the matrix instructions it runs on, six bf16
+MFMAs for an f32 product or f32 MFMAs; `peak` is their mean weighted by work),
+`roofline_mfma_all` for every MFMA kernel (GEMMs and fused attention); `cpu_baseline` is the CPU oracle (a C++ restatement of the reference's CPU
 evaluator, the reference itself being TypeScript that cannot run here) on this host's
 cores, on a bounded number of steps of the same workload.
 """
@@ -28,26 +29,28 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_F32_MFMA_TFLOPS = 157.3
+PEAK_SPLIT_BF16_TFLOPS = 2500.0 / 6   # f32 products as six bf16 ones
 PEAK_HBM_GBS = 8000.0
 RING = 8
 
 
 def family_rates(nodes, kms):
     """Per-family work and kernel time of one step from per-node kernel durations (ms):
-    GEMMs, convolutions and attention on the f32 MFMA roofline, the rest on HBM."""
+    GEMMs, convolutions and attention on the MFMA roofline (products on the split-bf16
+    tile at a sixth of the bf16 peak, all else at the f32 one), the rest on HBM."""
+    def least(n):   # us at peak
+        return n['flops'] / 1e6 / (PEAK_SPLIT_BF16_TFLOPS if n.get('tile', '').startswith('x3') else PEAK_F32_MFMA_TFLOPS)
+
+    def rates(sel):
+        f, t, us = sum(n['flops'] for n, _ in sel), sum(t for _, t in sel), sum(least(n) for n, _ in sel)
+        return {'flop_per_step': f, 'ms': t, 'tflops': f / max(t, 1e-12) / 1e9,
+                'peak_tflops': f / us / 1e6 if us else PEAK_F32_MFMA_TFLOPS, 'frac_mfma_peak': us / max(1e3 * t, 1e-12)}
     fam = {'gemm': ('gemm',), 'conv': ('conv',), 'attention': ('attention',)}
     out = {}
     for name, kinds in fam.items():
         sel = [(n, t) for n, t in zip(nodes, kms) if n['kind'] in kinds]
-        f = sum(n['flops'] for n, _ in sel)
-        t = sum(t for _, t in sel)
-        out[name] = {'flop_per_step': f, 'bytes_per_step': sum(n['bytes'] for n, _ in sel), 'launches': len(sel),
-                     'ms': t, 'tflops': f / max(t, 1e-12) / 1e9,
-                     'frac_f32_peak': f / max(t, 1e-12) / 1e9 / PEAK_F32_MFMA_TFLOPS}
-    mf = out['gemm']['flop_per_step'] + out['attention']['flop_per_step'] + out['conv']['flop_per_step']
-    mt = out['gemm']['ms'] + out['attention']['ms'] + out['conv']['ms']
-    out['mfma_all'] = {'flop_per_step': mf, 'ms': mt, 'tflops': mf / max(mt, 1e-12) / 1e9,
-                       'frac_f32_peak': mf / max(mt, 1e-12) / 1e9 / PEAK_F32_MFMA_TFLOPS}
+        out[name] = dict(rates(sel), bytes_per_step=sum(n['bytes'] for n, _ in sel), launches=len(sel))
+    out['mfma_all'] = rates([(n, t) for n, t in zip(nodes, kms) if n['kind'] in ('gemm', 'conv', 'attention')])
     sel = [(n, t) for n, t in zip(nodes, kms) if n['kind'] not in ('gemm', 'conv', 'attention')]
     b = sum(n['bytes'] for n, _ in sel)
     t = sum(t for _, t in sel)
@@ -153,11 +156,11 @@ def kernel_events(key, iters=20, warmup=20):
     for name in ('gemm', 'attention', 'conv'):
         f = fam[name]
         if f['launches']:
-            o.append(f"| {name} (f32 MFMA) | {f['launches']} | {1e3 * f['ms']:.1f} | {f['flop_per_step'] / 1e9:.3f} GFLOP | "
-                     f"{f['tflops']:.1f} TFLOP/s | {100 * f['frac_f32_peak']:.1f} % |")
+            o.append(f"| {name} | {f['launches']} | {1e3 * f['ms']:.1f} | {f['flop_per_step'] / 1e9:.3f} GFLOP | "
+                     f"{f['tflops']:.1f} TFLOP/s | {100 * f['frac_mfma_peak']:.1f} % of {f['peak_tflops']:.1f} |")
     m = fam['mfma_all']
     o.append(f"| all MFMA work | | {1e3 * m['ms']:.1f} | {m['flop_per_step'] / 1e9:.3f} GFLOP | {m['tflops']:.1f} TFLOP/s | "
-             f"{100 * m['frac_f32_peak']:.1f} % |")
+             f"{100 * m['frac_mfma_peak']:.1f} % of {m['peak_tflops']:.1f} |")
     ng = fam['non_gemm']
     o.append(f"| other launches (HBM) | {ng['launches']} | {1e3 * ng['ms']:.1f} | {ng['bytes_per_step'] / 1e6:.1f} MB | "
              f"{ng['gbs']:.0f} GB/s | {100 * ng['frac_hbm_peak']:.1f} % |")
@@ -397,7 +400,7 @@ def main():
         return
     if args.gpus != 1:
         print(json.dumps({'error': 'this build runs on one GPU per process; multi-GPU data parallelism is '
-                                   'designed (DESIGN.md) but not built, so --gpus must be 1'}))
+                                   'designed but not built, so --gpus must be 1'}))
         sys.exit(2)
     from tensorgrad_amd import backend, configs
     if backend.device_count() < 1:
@@ -442,10 +445,10 @@ def main():
         'config': {'workload': cfg.title, 'samples_per_step': cfg.samples_per_step, 'sample_unit': cfg.sample_unit,
                    'samples_per_s': round(head['samples_per_s'], 1),
                    'device_replay_ms_per_step': round(head['device_replay_ms'], 4)},
-        'roofline': {'bound': 'mfma', 'kernel': 'k_gemm (f32 MFMA GEMM family: every matmul / matmul_batched '
-                                                'launch of one step, split-K reductions included)',
-                     'achieved': round(g['tflops'], 3), 'peak': PEAK_F32_MFMA_TFLOPS, 'unit': 'TFLOP/s',
-                     'frac': round(g['frac_f32_peak'], 4),
+        'roofline': {'bound': 'mfma', 'kernel': 'k_gemm_x3, k_gemm_* (every matmul / matmul_batched launch of one step, '
+                                                'split-K reductions included)',
+                     'achieved': round(g['tflops'], 3), 'peak': round(g['peak_tflops'], 1), 'unit': 'TFLOP/s',
+                     'frac': round(g['frac_mfma_peak'], 4),
                      'traffic': profiled_traffic(os.path.join(ROOT, 'profiles', 'gemm_transformer_traffic.txt')),
                      'timing': 'kernel start/end events of each launch in eager steps (tg_profile_kernels)',
                      'launches_per_step': g['launches'],
@@ -453,8 +456,9 @@ def main():
                      'algorithmic_flop_per_launch': round(g['flop_per_step'] / max(g['launches'], 1)),
                      'algorithmic_bytes_per_launch': round(g['bytes_per_step'] / max(g['launches'], 1))},
         'roofline_mfma_all': {'bound': 'mfma', 'kernels': 'GEMMs + fused attention (+ convolutions)',
-                              'achieved': round(head['mfma_all']['tflops'], 3), 'peak': PEAK_F32_MFMA_TFLOPS,
-                              'unit': 'TFLOP/s', 'frac': round(head['mfma_all']['frac_f32_peak'], 4),
+                              'achieved': round(head['mfma_all']['tflops'], 3),
+                              'peak': round(head['mfma_all']['peak_tflops'], 1), 'unit': 'TFLOP/s',
+                              'frac': round(head['mfma_all']['frac_mfma_peak'], 4),
                               'flop_per_step': head['mfma_all']['flop_per_step']},
         'roofline_non_gemm': {'bound': 'hbm', 'achieved': round(head['non_gemm']['gbs'], 1), 'peak': PEAK_HBM_GBS,
                               'unit': 'GB/s', 'frac': round(head['non_gemm']['frac_hbm_peak'], 4),
@@ -465,10 +469,10 @@ def main():
                         'samples_per_s': round(r['samples_per_s'], 1), 'device_replay_ms': round(r['device_replay_ms'], 4),
                         'kernel_ms_per_step': round(r['kernel_ms_per_step'], 4),
                         'host_batch_steps_per_s': round(r['host_batch_steps_per_s'], 2),
-                        'gemm_tflops': round(r['gemm']['tflops'], 2), 'gemm_frac_f32_peak': round(r['gemm']['frac_f32_peak'], 4),
+                        'gemm_tflops': round(r['gemm']['tflops'], 2), 'gemm_frac_mfma_peak': round(r['gemm']['frac_mfma_peak'], 4),
                         'conv_tflops': round(r['conv']['tflops'], 2),
                         'attention_tflops': round(r['attention']['tflops'], 2),
-                        'mfma_all_frac_f32_peak': round(r['mfma_all']['frac_f32_peak'], 4),
+                        'mfma_all_frac_mfma_peak': round(r['mfma_all']['frac_mfma_peak'], 4),
                         'non_gemm_gbs': round(r['non_gemm']['gbs'], 1),
                         'non_gemm_frac_hbm': round(r['non_gemm']['frac_hbm_peak'], 4),
                         'launch_nodes': r['launch_nodes'], 'kinds': r['kinds'], 'top_gemms': r['gemm']['top']}

@@ -531,20 +531,22 @@ struct StoreC {   // (tile_finish stores it)
 // 2^-25 of the largest (mid * low, low * mid, low * low) are left out: six MFMAs in place of sixteen's worth of time.
 // Operands are scaled by 2^16 on the way, which puts the last bit of the smallest f32 (2^-149) on bf16's (2^-133): without
 // it the low terms of values below 2^-110 would be lost (2^-120: wrong by 2e-5). The sums are scaled back by 2^-32.
-// Accuracy against 64 bits is no worse than the f32 tile's over sums of many terms (norm-wise, K = 64 .. 4096: 0.7e-7 ..
-// 1.1e-7 against 1.4e-7 .. 1.7e-7; values of one sign 0.5e-7 .. 0.6e-7 against 1.1e-7 .. 0.5e-7): an MFMA adds 16 exact
-// bf16 products with one rounding where the f32 one adds two, and every 32 k go into a fresh accumulator (the small terms
-// first) that is added to the running sum. A sum that one of its terms makes up has that term's error, the products left
+// Accuracy against 64 bits is no worse than the f32 tile's over sums of many terms (norm-wise, K = 64 .. 65536: 0.7e-7 ..
+// 1.5e-7 against 1.3e-7 .. 2.1e-7; terms of one sign 0.3e-7 .. 0.8e-7 against 0.5e-7 .. 1.1e-7, only one unsplit sum over 2048 k
+// above, 0.65e-7 against 0.56e-7): an MFMA adds 16 exact bf16 products with one rounding where the f32 one adds two, and
+// every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum. A sum that one of its terms makes up has that term's error, the products left
 // out and the MFMA's rounding: up to 1.4 units in the last place (0.39 rms), where an f32 product rounds once (0.5, 0.29).
 // Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
 // are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile; so
 // do values and sums that the scale takes past the f32 range (2^112 and 2^96).
 //
-// What bounds it: per 16 k a wavefront with a 64 x 64 tile issues 24 MFMAs (32 cycles each) and about 130 vector
-// instructions (5.5 per element split, 2 per accumulator), and an MFMA keeps the vector port for half its time, so the
-// two together need about 1.4 of the MFMAs' own time; two blocks a CU hide each other's barriers and latencies. At
-// 4096^3 the matrix cores are 59 % busy at the 1.8 GHz the card then holds (187 TFLOP/s as f32 work, against 130 for
-// the f32 tile); [65536, 256] x [256, 256] 92 -> 58 us, [4000, 512] x [512, 2048] 88 -> 55 us.
+// What bounds it: per 16 k a wavefront with a 64 x 64 tile issues 24 MFMAs (32 cycles each) and about 150 vector
+// instructions (6.5 per element scaled and split, 2 per accumulator), and an MFMA keeps the vector port for half its time, so
+// the two together need about 1.5 of the MFMAs' own time; two blocks a CU hide each other's barriers and latencies. Over
+// [256, 65536] x [65536, 256] the matrix pipe is busy for 36 % of the launch, at 6.7 other vector instructions per MFMA,
+// of the [65536, 256] layers' products 32 % at 9 (K = 256: the first loads, the stores). Against the f32 tile: 4096^3 1018 -> 784 us
+// (135 -> 175 TFLOP/s as f32 work), [65536, 256] x [256, 256] 83 -> 59 us, [256, 65536] x [65536, 256] 83 -> 65 us,
+// [4000, 512] x [512, 2048] 79 -> 57 us.
 //
 // Tile: operands go through registers (loads three stages ahead of their use, split, then stored as three bf16 planes
 // into the other half of a double LDS buffer while this half is multiplied), so they need no alignment: a load is
@@ -732,7 +734,8 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, uint32_t b, const Epi
   // FRESH: the running sums take the last stages' part and a new one begins.
   // The bf16 MFMAs round towards one side by a little (2^-27 of a part), which over thousands of k of terms of either
   // sign would be most of the error. So every other part is made of a negated operand (the one of fewer rows), and the
-  // running sums change sign each time: [256, 65536] x [65536, 256] is 1.83e-7 from its f64 value so, 3.9e-7 without.
+  // running sums change sign each time: [256, 65536] x [65536, 256], its partials added in f32, was 1.83e-7 from its f64
+  // value so and 3.9e-7 without.
   constexpr bool SIGNA = TA::PER <= TB::PER;
   auto sign = [](int st) { return (st & 2) ? -1.0f : 1.0f; };
   auto body = [&](int st, auto ptag, auto ftag) {
