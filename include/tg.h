@@ -167,7 +167,8 @@ tg_status tg_safetensors_index(const void* buf, int64_t len, char* out_json, int
 
 /* ---- measurement (no reference counterpart) ---------------------------------------
  * Kernel-level schedule of the lowered step, as JSON: one entry per launch node with
- * its kind, shape summary, algorithmic FLOP and byte counts. */
+ * its kind, shape summary, algorithmic FLOP and byte counts, a fused group's operations
+ * ("ops") and a product's kernel ("tile"). */
 tg_status tg_describe(tg_runtime* rt, char* buf, int64_t buflen);
 /* Lower an IR document without touching the device (no allocation, no launches) and
  * write the same JSON schedule as tg_describe. Usable on a machine without a GPU. */
