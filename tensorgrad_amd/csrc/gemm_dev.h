@@ -532,10 +532,11 @@ struct StoreC {   // (tile_finish stores it)
 // Operands are scaled by 2^16 on the way, which puts the last bit of the smallest f32 (2^-149) on bf16's (2^-133): without
 // it the low terms of values below 2^-110 would be lost (2^-120: wrong by 2e-5). The sums are scaled back by 2^-32.
 // Accuracy against 64 bits is no worse than the f32 tile's over sums of many terms (norm-wise, K = 64 .. 65536: 0.7e-7 ..
-// 1.5e-7 against 1.3e-7 .. 2.1e-7; terms of one sign 0.3e-7 .. 0.8e-7 against 0.5e-7 .. 1.1e-7, only one unsplit sum over 2048 k
-// above, 0.65e-7 against 0.56e-7): an MFMA adds 16 exact bf16 products with one rounding where the f32 one adds two, and
-// every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum. A sum that one of its terms makes up has that term's error, the products left
-// out and the MFMA's rounding: up to 1.4 units in the last place (0.39 rms), where an f32 product rounds once (0.5, 0.29).
+// 1.5e-7 against 1.3e-7 .. 2.1e-7; terms of one sign 0.3e-7 .. 0.8e-7 against 0.5e-7 .. 1.1e-7, only one unsplit sum over
+// 2048 k above, 0.65e-7 against 0.56e-7): an MFMA adds 16 exact bf16 products with one rounding where the f32 one adds two,
+// and every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum. A sum that one of
+// its terms makes up has that term's error, the products left out and the MFMA's rounding: up to 1.4 units in the last
+// place (0.39 rms), where an f32 product rounds once (0.5, 0.29).
 // Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
 // are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile; so
 // do values and sums that the scale takes past the f32 range (2^112 and 2^96).
@@ -543,10 +544,10 @@ struct StoreC {   // (tile_finish stores it)
 // What bounds it: per 16 k a wavefront with a 64 x 64 tile issues 24 MFMAs (32 cycles each) and about 150 vector
 // instructions (6.5 per element scaled and split, 2 per accumulator), and an MFMA keeps the vector port for half its time, so
 // the two together need about 1.5 of the MFMAs' own time; two blocks a CU hide each other's barriers and latencies. Over
-// [256, 65536] x [65536, 256] the matrix pipe is busy for 36 % of the launch, at 6.7 other vector instructions per MFMA,
-// of the [65536, 256] layers' products 32 % at 9 (K = 256: the first loads, the stores). Against the f32 tile: 4096^3 1018 -> 784 us
-// (135 -> 175 TFLOP/s as f32 work), [65536, 256] x [256, 256] 83 -> 59 us, [256, 65536] x [65536, 256] 83 -> 65 us,
-// [4000, 512] x [512, 2048] 79 -> 57 us.
+// [256, 65536] x [65536, 256] the matrix pipe is busy for 36 % of the launch, at 6.7 other vector instructions per MFMA; over
+// [65536, 256] x [256, 256] for 32 %, at 9 (short K: the first loads, the stores). Against the f32 tile: 4096^3
+// 1018 -> 784 us (135 -> 175 TFLOP/s as f32 work), [65536, 256] x [256, 256] 83 -> 59 us, [256, 65536] x [65536, 256]
+// 83 -> 65 us, [4000, 512] x [512, 2048] 79 -> 57 us.
 //
 // Tile: operands go through registers (loads three stages ahead of their use, split, then stored as three bf16 planes
 // into the other half of a double LDS buffer while this half is multiplied), so they need no alignment: a load is

@@ -385,7 +385,8 @@ struct XPlan { int tiling, splits; int64_t kps; double us; };
 constexpr int64_t kXSplitBytes = (16 << 20) - (512 << 10);
 
 // The tiling (and for K >= 1024 the split of K, partial products added by k_splitk_reduce) with the least time by the
-// figures above. A product with K under 1024 is never split, so its epilogue group can run in it.
+// figures above. A product with K under 1024 is never split, so its epilogue group can run in it. Over 150 products with M,
+// N and K drawn from 64 .. 8192, 64 .. 4096 and 32 .. 8192 the chosen plans take 0.50 to 1.04 of the f32 tiles' time.
 XPlan x3_plan(const GemmDesc& d) {
   XPlan best{-1, 1, d.K, 0.0};
   const int64_t range = x3_range(d);
@@ -911,9 +912,9 @@ std::string gemm_cat_tile(const GemmDesc& d, const GemmCat& c) { return cat_x3(d
 // Segments of whole 16-k stages run on the split-bf16 tile, unsplit.
 static bool sum_x3(const GemmDesc& all, int64_t seg) { return seg % kXK == 0 && x3_ok(all); }
 
-// Whether a sum runs as one unsplit launch over all of its terms' k: always below 1024 k (a launch or two less, at most
-// 10 us longer), from there where that is estimated no longer than the products apart (grouped in one launch, or split over
-// K) with an addition that reads them and writes the sum at 4 TB/s. Steps in us, in one launch and apart: 2 x [8000, 1024] x
+// Whether a sum runs as one unsplit launch over all of its terms' k: always below 1024 k (a launch or two less), from there
+// where that is estimated no longer than the products apart (grouped in one launch, or split over K) with an addition
+// that reads them and writes the sum at 4 TB/s. Steps in us, in one launch and apart: 2 x [8000, 1024] x
 // [1024, 384] 99 and 115, 3 x [1600, 512] x [512, 512] 39 and 42; but 3 x [108, 384] x [384, 384] 32 and 21, 2 x [512, 1024]
 // x [1024, 512] 45 and 37, 2 x [4096, 2048] x [2048, 512] 128 and 111, 2 x [128, 8192] x [8192, 256] 239 and 33. A sum that
 // would be longer than its error allows (x3_group_tiling) stays apart.
