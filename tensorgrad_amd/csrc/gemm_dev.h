@@ -536,7 +536,8 @@ struct StoreC {   // (tile_finish stores it)
 // 2048 k above, 0.65e-7 against 0.56e-7): an MFMA adds 16 exact bf16 products with one rounding where the f32 one adds two,
 // and every 32 k go into a fresh accumulator (the small terms first) that is added to the running sum. A sum that one of
 // its terms makes up has that term's error, the products left out and the MFMA's rounding: up to 1.4 units in the last
-// place (0.39 rms), where an f32 product rounds once (0.5, 0.29).
+// place (0.39 rms), where an f32 product rounds once (0.5, 0.29). With mid * low and low * mid it would be 1.0 (0.39 rms) and
+// sums of many terms the same, for steps 6 to 10 % longer.
 // Infinities: inf * b must be inf, but splits into inf * b_hi + inf * b_mid + .., which is NaN. A wavefront whose sums
 // are not all finite multiplies its tile again with f32 MFMAs (x3_redo), so such values come out as from the f32 tile; so
 // do values and sums that the scale takes past the f32 range (2^112 and 2^96).
